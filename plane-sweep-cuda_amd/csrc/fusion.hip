@@ -23,6 +23,7 @@
 #include "psw_common.h"
 #include "rn_math.h"
 
+#include <cmath>
 #include <type_traits>
 #include <vector>
 
@@ -93,57 +94,201 @@ __device__ inline int vote_bin(const Cam& cam, const float* __restrict__ depth, 
     return (int)fmaxf(q, 0.f);
 }
 
-__global__ void fusion_hist_kernel(FusionView f, Cam cam, const float* __restrict__ depth, int W, int H, float thr) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    const int y = blockIdx.y * blockDim.y + threadIdx.y;
-    const int z = blockIdx.z;
-    if (x >= f.w || y >= f.h || z >= f.d) return;
-    float cx, cy, cz;
-    voxel_centre(f, x, y, z, cx, cy, cz);
-    const int bin = vote_bin(cam, depth, W, H, thr, cx, cy, cz);
-    if (bin < 0) return;
-    const size_t i = ((size_t)z * f.h + y) * f.w + x;
-    f.hist[i * FB + bin] = (uint16_t)(f.hist[i * FB + bin] + 1);
-}
-
-constexpr int FH_BATCH = 24;  // depthmaps per launch (kernel-argument space)
+constexpr int FH_BATCH = 40;  // depthmaps per launch (kernel-argument space; at most 64, one lane each)
 
 struct CamBatch {
     Cam cam[FH_BATCH];
     int m;
 };
 
+// False only if no voxel centre of the box with centre c and half extents e
+// can pass vote_bin's image test for this camera.  In image coordinates
+// k = K (R c + T) is affine in c, and px = k0 / k2 is left of the image
+// where k0 and k2 have opposite signs and right of it where k0 - (W-1) k2 has
+// k2's sign (rows alike), so each is decided by the range of an affine
+// function over the box, once k2 keeps one sign over it.  (A voxel behind
+// the camera can project into the image, and votes.)  The margins, 2^-16 of
+// the sum of the terms' magnitudes, are hundreds of times the float rounding
+// of k here and in vote_bin.  A box that is not clearly outside is seen;
+// comparisons with NaN are false, so it is seen too.
+__device__ inline bool box_seen(const Cam& cam, int W, int H, const float (&c)[3], const float (&e)[3]) {
+    float f[3], A[3][3], S[3];   // k at the centre, its gradient, its terms' magnitude over the box
+    float rc[3], rm[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const float* R = &cam.R.m[3 * i];
+        const float t = i == 0 ? cam.T.x : i == 1 ? cam.T.y : cam.T.z;
+        rc[i] = R[0] * c[0] + R[1] * c[1] + R[2] * c[2] + t;
+        rm[i] = fabsf(R[0]) * (fabsf(c[0]) + e[0]) + fabsf(R[1]) * (fabsf(c[1]) + e[1]) +
+                fabsf(R[2]) * (fabsf(c[2]) + e[2]) + fabsf(t);
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const float* K = &cam.K.m[3 * i];
+        f[i] = K[0] * rc[0] + K[1] * rc[1] + K[2] * rc[2];
+        S[i] = 0x1p-16f * (fabsf(K[0]) * rm[0] + fabsf(K[1]) * rm[1] + fabsf(K[2]) * rm[2]);
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            A[i][j] = K[0] * cam.R.m[j] + K[1] * cam.R.m[3 + j] + K[2] * cam.R.m[6 + j];
+    }
+    auto reach = [&](float a, float b, float d) { return fabsf(a) * e[0] + fabsf(b) * e[1] + fabsf(d) * e[2]; };
+    const float r2 = reach(A[2][0], A[2][1], A[2][2]) + S[2];
+    const bool front = f[2] - r2 > 0.f, behind = f[2] + r2 < 0.f;
+    bool outside = false;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const float n = (float)((i == 0 ? W : H) - 1);
+        const float lo = f[i], rlo = reach(A[i][0], A[i][1], A[i][2]) + S[i];
+        const float hi = f[i] - n * f[2];
+        const float rhi = reach(A[i][0] - n * A[2][0], A[i][1] - n * A[2][1], A[i][2] - n * A[2][2]) + S[i] + n * S[2];
+        outside |= front && (lo + rlo < 0.f || hi - rhi > 0.f);
+        outside |= behind && (lo - rlo > 0.f || hi + rhi < 0.f);
+    }
+    return !outside;
+}
+
 // Votes of up to FH_BATCH depthmaps per voxel, counted in registers and added
 // to the stored histogram once.  Counts are integers, so the order of the
 // votes does not matter and the result equals m single updates (mod 2^16).
-__global__ void fusion_hist_batch_kernel(FusionView f, CamBatch cb, const float* __restrict__ depths, int W, int H,
-                                         float thr) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    const int y = blockIdx.y * blockDim.y + threadIdx.y;
-    const int z = blockIdx.z;
-    if (x >= f.w || y >= f.h || z >= f.d) return;
-    float cx, cy, cz;
-    voxel_centre(f, x, y, z, cx, cy, cz);
-    uint32_t cnt[FB];
+//
+// Most cameras do not see a given voxel, and the projection has no fused or
+// approximate step.  So each wave owns a box of 16 x 4 x 4 voxels (four z
+// per lane; a row of it is 256 bytes of histogram; 8 x 8 and 32 x 2 boxes
+// were 14 % and 6 % slower), its lanes first test one camera each against
+// the box, and the wave then projects into the cameras that may see it, read
+// as scalars.  The four votes of a lane are branch-free, so that their loads
+// are in flight together: a voxel outside the image reads pixel 0 and adds
+// nothing.  What is left is bound by the gathers (about 40 cache accesses
+// per wave load, address unit busy 77 % of the time): the two neighbours of
+// an image row come in one 8-byte load (1.21 ms with one load each).
+// Their results are vote_bin's, bit for bit:
+//   - operands of the projective divide between 2^-40 and 2^40 (else the
+//     wave takes vote_bin) need one reciprocal and two residual corrections
+//     per quotient (div_nr: scaling by powers of two is exact, so its range
+//     |x| <= d is no restriction);
+//   - the bin's quotient has 2^-25 thr <= x <= 2 thr and the same treatment;
+//   - its value q is in [1, 6], where x + 1/2 is exact below each half, so
+//     truncation rounds like roundf; NaN takes the upper bin through fminf;
+//   - PINHOLE (K of the usual form, last row 0 0 1, no skew; finite centres):
+//     the products with K's zeros are zeros, which change no sum;
+//   - a voxel's counts of one launch fit bytes: a vote is a shift and an add.
+// `general` (set by the host: K, R, T or the threshold outside those ranges,
+// images of 2^29 pixels or one column) sends every wave to vote_bin.
+// The stored histogram is read and written only where there are votes.
+// 50 depthmaps of 640 x 480 on a ring (29 % of the projections land), 256^3
+// voxels: 0.84 ms, against 1.83 ms with every voxel projected into every
+// camera, one voxel per lane.
+constexpr int FH_X = 16, FH_Y = 4, FH_Z = 4;
+
+struct __attribute__((packed, aligned(4))) Pair {
+    float a, b;   // neighbours of one image row, one load
+};
+
+template <bool PINHOLE>
+__global__ __launch_bounds__(256) void fusion_hist_batch_kernel(FusionView f, CamBatch cb,
+                                                                const float* __restrict__ depths, int W, int H,
+                                                                float thr, bool general) {
+    const int lane = threadIdx.x & 63;
+    const int x0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * FH_X, y0 = blockIdx.y * FH_Y, z0 = blockIdx.z * FH_Z;
+    if (x0 >= f.w) return;
+    const int x = x0 + (lane & (FH_X - 1)), y = y0 + lane / FH_X;
+    float cx, cy, cl, cz[FH_Z];
+    voxel_centre(f, x, y, z0 + (lane & (FH_Z - 1)), cx, cy, cl);
 #pragma unroll
-    for (int k = 0; k < FB; ++k) cnt[k] = 0;
+    for (int v = 0; v < FH_Z; ++v) cz[v] = __shfl(cl, v);
+    const float ax = __shfl(cx, 0), bx = __shfl(cx, FH_X - 1), ay = __shfl(cy, 0), by = __shfl(cy, 63);
+    bool seen = false;
+    if (lane < cb.m) {
+        const float c[3] = {0.5f * (ax + bx), 0.5f * (ay + by), 0.5f * (cz[0] + cz[FH_Z - 1])};
+        const float e[3] = {0.5f * fabsf(bx - ax), 0.5f * fabsf(by - ay), 0.5f * fabsf(cz[FH_Z - 1] - cz[0])};
+        seen = box_seen(cb.cam[lane], W, H, c, e);
+    }
+    unsigned long long todo = __ballot(seen);
+    const bool live = x < f.w && y < f.h;
     const size_t plane = (size_t)W * H;
-    for (int j = 0; j < cb.m; ++j) {
-        const int bin = vote_bin(cb.cam[j], depths + (size_t)j * plane, W, H, thr, cx, cy, cz);
+    const float fw = (float)(W - 1), fh = (float)(H - 1);
+    const float span = 2.f * thr, rspan = rcp_nr(span);
+    uint32_t lo[FH_Z] = {}, hi[FH_Z] = {};   // counts of bins 0..3 and 4..7, a byte each
+    auto count = [&](int v, bool ok, int bin) {
+        const uint32_t one = ok ? 1u << (8 * (bin & 3)) : 0u;
+        lo[v] += bin < 4 ? one : 0u;
+        hi[v] += bin < 4 ? 0u : one;
+    };
+    while (todo) {
+        const int j = __builtin_ctzll(todo);
+        todo &= todo - 1;
+        const float* __restrict__ depth = depths + (size_t)j * plane;
+        const Cam& cam = cb.cam[j];
+        float k[FH_Z][3];
+        float mn = __builtin_inff(), mx = 0.f;
 #pragma unroll
-        for (int k = 0; k < FB; ++k) cnt[k] += (bin == k) ? 1u : 0u;
-    }
-    const size_t i = ((size_t)z * f.h + y) * f.w + x;
-    uint4* hp = reinterpret_cast<uint4*>(f.hist + i * FB);
-    uint4 h = *hp;
-    uint32_t w4[4] = {h.x, h.y, h.z, h.w};
+        for (int v = 0; v < FH_Z; ++v) {
+            float c0, c1, c2;
+            mv3(cam.R, cx, cy, cz[v], c0, c1, c2);
+            c0 = c0 + cam.T.x; c1 = c1 + cam.T.y; c2 = c2 + cam.T.z;
+            if constexpr (PINHOLE) {
+                k[v][0] = cam.K.m[0] * c0 + cam.K.m[2] * c2;
+                k[v][1] = cam.K.m[4] * c1 + cam.K.m[5] * c2;
+                k[v][2] = c2;
+            } else {
+                mv3(cam.K, c0, c1, c2, k[v][0], k[v][1], k[v][2]);
+            }
+            mn = fminf(mn, fminf(fminf(fabsf(k[v][0]), fabsf(k[v][1])), fabsf(k[v][2])));
+            mx = fmaxf(mx, fmaxf(fmaxf(fabsf(k[v][0]), fabsf(k[v][1])), fabsf(k[v][2])));
+        }
+        if (general || __any(!(mn >= 0x1p-40f && mx <= 0x1p40f))) {
+#pragma unroll 1
+            for (int v = 0; v < FH_Z; ++v) {
+                const float z = v == 0 ? cz[0] : v == 1 ? cz[1] : v == 2 ? cz[2] : cz[3];
+                const int bin = vote_bin(cam, depth, W, H, thr, cx, cy, z);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const uint32_t lo = (w4[k] + cnt[2 * k]) & 0xffffu;
-        const uint32_t hi = ((w4[k] >> 16) + cnt[2 * k + 1]) & 0xffffu;
-        w4[k] = lo | (hi << 16);
+                for (int u = 0; u < FH_Z; ++u) count(u, u == v && bin >= 0, bin);
+            }
+            continue;
+        }
+        bool in[FH_Z];
+        float fx[FH_Z], fy[FH_Z], d00[FH_Z], d01[FH_Z], d10[FH_Z], d11[FH_Z];
+#pragma unroll
+        for (int v = 0; v < FH_Z; ++v) {
+            const float r = rcp_nr(k[v][2]);
+            const float px = div_nr(k[v][0], k[v][2], r), py = div_nr(k[v][1], k[v][2], r);
+            in[v] = px >= 0.f && px <= fw && py >= 0.f && py <= fh;
+            const uint32_t iy = (uint32_t)py;
+            const bool last = !(px < fw);           // px == W - 1: both neighbours are the last column
+            const uint32_t ix = (uint32_t)px - (last ? 1u : 0u);
+            const uint32_t o = in[v] ? 4u * (iy * (uint32_t)W + ix) : 0u;
+            const uint32_t o1 = in[v] && py < fh ? o + 4u * (uint32_t)W : o;
+            fx[v] = __builtin_amdgcn_fractf(px);
+            fy[v] = __builtin_amdgcn_fractf(py);
+            const char* b = reinterpret_cast<const char*>(depth);
+            const Pair r0 = *reinterpret_cast<const Pair*>(b + o), r1 = *reinterpret_cast<const Pair*>(b + o1);
+            d00[v] = last ? r0.b : r0.a;
+            d01[v] = r0.b;
+            d10[v] = last ? r1.b : r1.a;
+            d11[v] = r1.b;
+        }
+#pragma unroll
+        for (int v = 0; v < FH_Z; ++v) {
+            const float l0 = d00[v] + fy[v] * (d10[v] - d00[v]), l1 = d01[v] + fy[v] * (d11[v] - d01[v]);
+            const float sd = l0 + fx[v] * (l1 - l0) - k[v][2];
+            const float q = fminf(div_nr(sd + thr, span, rspan) * (float)(FB - 3) + 1.f + 0.5f, (float)(FB - 2) + 0.5f);
+            count(v, in[v], sd >= thr ? FB - 1 : sd <= -thr ? 0 : (int)q);
+        }
     }
-    *hp = make_uint4(w4[0], w4[1], w4[2], w4[3]);
+    if (!live) return;
+#pragma unroll
+    for (int v = 0; v < FH_Z; ++v) {
+        if (z0 + v >= f.d || (lo[v] | hi[v]) == 0u) continue;
+        uint4* hp = reinterpret_cast<uint4*>(f.hist + (((size_t)(z0 + v) * f.h + y) * f.w + x) * FB);
+        const uint4 h = *hp;
+        uint32_t w4[4] = {h.x, h.y, h.z, h.w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t c2 = (k < 2 ? lo[v] : hi[v]) >> (16 * (k & 1));
+            w4[k] = ((w4[k] + (c2 & 0xffu)) & 0xffffu) | (((w4[k] >> 16) + ((c2 >> 8) & 0xffu)) << 16);
+        }
+        *hp = make_uint4(w4[0], w4[1], w4[2], w4[3]);
+    }
 }
 
 // ---- primal-dual ----------------------------------------------------------
@@ -873,6 +1018,39 @@ static Cam cam_of(const float* K, const float* R, const float* T) {
     return c;
 }
 
+// Votes of m depthmaps, in launches of equal size.
+static int hist_launch(const FusionView& f, const float* depths, int m, int W, int H, const float* K, const float* R,
+                       const float* T, float thr, hipStream_t st) {
+    const dim3 grd((unsigned)((f.w + 4 * FH_X - 1) / (4 * FH_X)), (unsigned)((f.h + FH_Y - 1) / FH_Y),
+                   (unsigned)((f.d + FH_Z - 1) / FH_Z));
+    // what fusion_hist_batch_kernel's shortcuts ask of the inputs
+    auto moderate = [](const float* p, int n) {
+        for (int i = 0; i < n; ++i)
+            if (!(std::fabs(p[i]) <= 0x1p18f)) return false;
+        return true;
+    };
+    bool general = !(thr >= 0x1p-18f && thr <= 0x1p18f) || W < 2 || (size_t)W * H >= (1u << 29) || !moderate(f.a, 3) ||
+                   !moderate(f.b, 3) || !moderate(R, 9 * m) || !moderate(T, 3 * m) || !moderate(K, 9 * m);
+    bool pinhole = !general;
+    for (int j = 0; j < m && pinhole; ++j) {
+        const float* k = K + 9 * j;
+        pinhole = k[1] == 0.f && k[3] == 0.f && k[6] == 0.f && k[7] == 0.f && k[8] == 1.f;
+    }
+    const int n = (m + FH_BATCH - 1) / FH_BATCH;
+    for (int k = 0; k < n; ++k) {
+        const int j0 = (int)((long)m * k / n), j1 = (int)((long)m * (k + 1) / n);
+        CamBatch cb;
+        cb.m = j1 - j0;
+        for (int j = j0; j < j1; ++j) cb.cam[j - j0] = cam_of(K + 9 * j, R + 9 * j, T + 3 * j);
+        const float* d = depths + (size_t)j0 * W * H;
+        if (pinhole) fusion_hist_batch_kernel<true><<<grd, 256, 0, st>>>(f, cb, d, W, H, thr, general);
+        else fusion_hist_batch_kernel<false><<<grd, 256, 0, st>>>(f, cb, d, W, H, thr, general);
+        const int s = launch_status("fusion_hist_batch_kernel");
+        if (s != PSW_OK) return s;
+    }
+    return PSW_OK;
+}
+
 }  // namespace psw
 
 using namespace psw;
@@ -928,10 +1106,7 @@ int psw_fusion_update_histogram(const psw_fusion_grid* g, const float* d_depthma
     PSW_CHECK_ARG(!(threshold < 0.f), "threshold must not be negative");
     PSW_CHECK_ARG(d_depthmap && K && R && T, "NULL pointer");
     PSW_CHECK_ARG(width >= 1 && height >= 1, "bad depthmap size");
-    const FusionView f = view_of(g);
-    const dim3 blk(64, 4, 1);
-    fusion_hist_kernel<<<vox_grid(f, blk), blk, 0, S(s)>>>(f, cam_of(K, R, T), d_depthmap, width, height, threshold);
-    return launch_status("fusion_hist_kernel");
+    return hist_launch(view_of(g), d_depthmap, 1, width, height, K, R, T, threshold, S(s));
 }
 
 int psw_fusion_update_histogram_batch(const psw_fusion_grid* g, const float* d_depthmaps, int m, int width, int height,
@@ -942,18 +1117,7 @@ int psw_fusion_update_histogram_batch(const psw_fusion_grid* g, const float* d_d
     PSW_CHECK_ARG(!(threshold < 0.f), "threshold must not be negative");
     PSW_CHECK_ARG(d_depthmaps && K && R && T, "NULL pointer");
     PSW_CHECK_ARG(m >= 0 && width >= 1 && height >= 1, "bad depthmap batch");
-    const FusionView f = view_of(g);
-    const dim3 blk(64, 4, 1);
-    for (int j0 = 0; j0 < m; j0 += FH_BATCH) {
-        CamBatch cb;
-        cb.m = std::min(FH_BATCH, m - j0);
-        for (int j = 0; j < cb.m; ++j) cb.cam[j] = cam_of(K + 9 * (j0 + j), R + 9 * (j0 + j), T + 3 * (j0 + j));
-        fusion_hist_batch_kernel<<<vox_grid(f, blk), blk, 0, S(s)>>>(f, cb, d_depthmaps + (size_t)j0 * width * height,
-                                                                     width, height, threshold);
-        st = launch_status("fusion_hist_batch_kernel");
-        if (st != PSW_OK) return st;
-    }
-    return PSW_OK;
+    return hist_launch(view_of(g), d_depthmaps, m, width, height, K, R, T, threshold, S(s));
 }
 
 int psw_fusion_update_u(const psw_fusion_grid* g, double tau, double lambda, psw_stream_t s) {

@@ -1,0 +1,56 @@
+"""Fusion histogram votes over the forms the kernel treats apart: grids that
+cut its 16 x 4 x 4 boxes, cameras inside, beside and behind the volume (whole
+boxes are skipped only when no voxel of them can project into the image; a
+voxel behind the camera can), voxels at the camera's own position (0 / 0), K with and without skew,
+depths that are not finite, a zero threshold, one-pixel images, and batches of one, just over one and over two launches.
+Whole numbers, compared exactly with the oracle."""
+import numpy as np
+import pytest
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+VOL = np.array([-1.0, -1.5, -2.0, 1.0, 1.5, 2.0], np.float32)
+
+
+def _cameras(rng, m, W, H, skew):
+    """Random poses: on the volume's axis, inside it, and far outside."""
+    from psw_amd import scene
+    K = np.array([[0.8 * W, skew, 0.5 * (W - 1)], [0.0, 0.9 * H, 0.5 * (H - 1)], [0.0, 0.0, 1.0]], np.float32)
+    Rs, ts = [], []
+    for j in range(m):
+        R = scene.rotation(rng.normal(size=3), rng.uniform(0.0, np.pi)) if j % 4 else np.eye(3)
+        C = rng.normal(size=3) * (0.0, 0.5, 1.0, 4.0)[j % 4]
+        Rs.append(R)
+        ts.append(-R @ C)
+    return K, np.array(Rs, np.float32), np.array(ts, np.float32)
+
+
+@pytest.mark.parametrize("grid,m,size,thr,skew", [
+    ((1, 1, 1), 3, (5, 4), 0.3, 0.0), ((17, 5, 3), 41, (33, 21), 0.25, 0.0), ((65, 4, 9), 81, (64, 48), 0.1, 3.0),
+    ((15, 17, 21), 9, (1, 7), 0.5, 0.0), ((79, 33, 31), 12, (160, 120), 0.0, 0.0), ((129, 9, 33), 2, (97, 3), 2.0, 0.0),
+    ((80, 60, 70), 17, (160, 120), 0.3, 0.0), ((80, 60, 70), 17, (160, 120), 0.01, 5.0)])
+def test_votes_match_oracle(gpu, grid, m, size, thr, skew):
+    from psw_amd import stages
+    from psw_amd.device import DeviceArray
+    (gw, gh, gd), (W, H) = grid, size
+    rng = np.random.default_rng(gw * 1000 + m)
+    K, R, T = _cameras(rng, m, W, H, skew)
+    depths = rng.uniform(0.2, 5.0, (m, H, W)).astype(np.float32)
+    for bad in (np.nan, np.inf, -np.inf, 0.0):
+        depths[rng.random(depths.shape) < 0.01] = bad
+    exp = np.zeros((gd, gh, gw, 8), np.uint16)
+    for j in range(m):
+        oracle.fusion_hist(exp, VOL, depths[j], K, R[j], T[j], thr)
+    print(f"[case] votes grid {grid} m {m} image {size} threshold {thr}: {int(exp.sum())} votes", flush=True)
+    assert 0 < int(exp.sum()) < m * gw * gh * gd
+    f = stages.Fusion(gw, gh, gd, VOL)
+    d = DeviceArray.from_host(depths)
+    K9 = np.tile(K, (m, 1, 1))
+    f.update_histogram_batch(d, m, W, H, K9, R, T, thr)
+    assert np.array_equal(f.download()["hist"], exp)
+    f.clear()
+    for j in range(m):
+        f.update_histogram(d.view(j), W, H, K, R[j], T[j], thr)
+    assert np.array_equal(f.download()["hist"], exp)
