@@ -248,7 +248,9 @@ int psw_sweep_homographies(float* d_H, const float* d_depths, int nplanes, int n
  * per source the best NCC over planes (strict >, zero start), depth averaged
  * over sources whose best NCC > nccthresh, zfar where none.  1-based pixel
  * convention.  d_H [nsrc][nplanes][9], d_depths [nplanes].  Bit-identical to
- * the reference's float arithmetic (no FMA contraction). */
+ * the reference's float arithmetic (no FMA contraction).  The sources' best
+ * values, 8 bytes per pixel and source, go to the library's workspace pool;
+ * under stream capture the call allocates nothing (and is slower). */
 int psw_sweep_fused_reference(const float* d_ref, const float* d_src, int width, int height, int nsrc,
                               const float* d_H, const float* d_depths, int nplanes, int winsize,
                               float stdthresh, float nccthresh, float zfar, float* d_depth_out, psw_stream_t s);
@@ -258,11 +260,11 @@ int psw_sweep_fused_reference(const float* d_ref, const float* d_src, int width,
  * coord_offset 0 = 0-based pixel convention, 1 = the reference's 1-based one.
  * fast = 0: reference-order arithmetic (bit-identical to the float oracle);
  * fast = 1: running window sums, reciprocal scaling and FMA.  With more
- * than one plane group (the default below about 9600 tiles of 32 x 16
- * pixels; PSW_SWEEP_GROUPS sets it) the groups' keys, 16 bytes per pixel,
- * come from the library's stream-ordered
- * workspace pool, which keeps freed blocks for later calls until the
- * process ends. */
+ * than one plane group (the default below about 3400 tiles of 1024 pixels;
+ * PSW_SWEEP_GROUPS sets it) the groups' results, 12 bytes per pixel and
+ * group up to 32 MiB in all, else keys of 16 bytes per pixel, go to the
+ * library's stream-ordered workspace pool, which keeps freed blocks for
+ * later calls until the process ends. */
 int psw_sweep_fused_aggregate(const float* d_ref, const float* d_src, int width, int height, int nsrc,
                               const float* d_H, int nplanes, int winsize, float stdthresh, int coord_offset,
                               int fast, int32_t* d_argmin, float* d_cost_min, float* d_cost_second,
@@ -275,7 +277,7 @@ int psw_sweep_argmin_depth(float* d_depth, const int32_t* d_argmin, const float*
 /* psw_sweep_fused_aggregate without any device allocation.  No counterpart
  * in the reference: for callers that cannot allocate device memory (code
  * under hipGraph capture, tight serving loops).  The plane groups'
- * per-pixel keys (16 bytes per pixel at any group count) go to a static
+ * results (as above: at most 32 MiB, or 16 bytes per pixel) go to a static
  * device array of PSW_SWEEP_SCRATCH_BYTES (32 MiB, held by every GPU the
  * library runs on until the process ends: frames up to 2^21 pixels) instead
  * of a per-call allocation; outputs are bit-identical to

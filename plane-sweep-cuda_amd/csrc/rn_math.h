@@ -1,6 +1,7 @@
 // rn_math.h -- correctly rounded square root and division for the
 // unit-ball projections of the primal-dual kernels (TGV2 duals in
-// tgv_point.h, fusion duals in fusion.hip).
+// tgv_point.h, fusion duals in fusion.hip), for the votes of fusion.hip and
+// for the reference-order sweep (sweep_fused.hip).
 #pragma once
 
 namespace psw {
@@ -40,6 +41,17 @@ __device__ __forceinline__ float div_nr(float x, float d, float y) {
     const float q0 = x * y;
     const float q1 = __builtin_fmaf(__builtin_fmaf(-d, q0, x), y, q0);
     return __builtin_fmaf(__builtin_fmaf(-d, q1, x), y, q1);
+}
+
+// s / WIN, correctly rounded, for |s| in [2^-60, 2^60]: one residual
+// correction of s * RN(1 / WIN) (checked against '/' for every mantissa and
+// every window size).
+template <int WIN>
+__device__ __forceinline__ float div_win(float s) {
+    if constexpr (WIN == 1) return s;
+    constexpr float r = 1.f / (float)WIN;
+    const float q = s * r;
+    return __builtin_fmaf(__builtin_fmaf(-q, (float)WIN, s), r, q);
 }
 
 // True when div_nr(x_i, sqrt(s), .) is exact for every |x_i| >= m.

@@ -1,13 +1,13 @@
 // sweep_fused.hip -- fused plane sweep for gfx950.
 //
-// One workgroup owns a 32x16 tile of reference pixels and sweeps every
+// One workgroup owns a tile of 1024 reference pixels and sweeps every
 // (plane, source) pair over it without leaving the CU:
 //   warp   : homography + bilinear sample of the source on the tile plus a
 //            window-radius halo, into LDS (reflect-101 halo positions, as the
 //            reference's box filters, kernels.cu:203-204 / :228-229);
 //   column : per column, register-blocked sums of I, I^2 and Ref*I over the
-//            window (4 output rows per thread), into LDS;
-//   row    : per pixel pair, sums of the column means -> mean, E[I^2],
+//            window (8 output rows per thread), into LDS;
+//   row    : per 4 pixels, sums of the column sums -> mean, E[I^2],
 //            E[Ref*I] -> std, NCC (kernels.cu:46-64, :103-120), reduction.
 // The reference instead writes eleven full-frame images to HBM per
 // (plane, source) (src/planesweep.cpp:206-249).
@@ -22,26 +22,27 @@
 // With FAST=false every sum, product and quotient is taken in the reference's
 // order (column mean = sum/win, row mean of column means = sum/win), so the
 // NCC is bit-identical to the reference's float arithmetic.  FAST=true
-// multiplies by 1/win, keeps running window sums down each column segment
-// (TY/4 rows) and along each row's pixels, and uses explicit fused
+// multiplies by 1/win, keeps running window sums down groups of 4 rows of a
+// column and along pairs of a row's pixels, and uses explicit fused
 // multiply-adds and the hardware reciprocal: its results are the same in
-// every launch of one tile height (single frame, batched, any plane groups),
-// and differ in the last bits between tile heights.
+// every launch (single frame, batched, any plane groups, either tile shape).
 #include "psw_common.h"
+#include "rn_math.h"
 
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 namespace psw {
 
-// Tile: SW_TX x TY pixels, TY = 16 or 32 (a template parameter; the
-// aggregated sweep's launches choose it, the reference reduction uses 16).
-// A taller tile warps fewer halo positions per pixel (the window radius is
-// added on all four sides) and gives the row pass more pixels per thread.
-constexpr int SW_TX = 32;       // tile width  (pixels)
-constexpr int SW_TY = 16;       // default tile height (pixels)
+// Tile: 64 x 16 or 32 x 32 pixels (template parameters; the launch chooses).
+// Both are 1024 pixels, 4 per thread of a row pass.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
 constexpr int SW_THREADS = 256; // 4 waves
-constexpr int SW_NCG = 4;       // column-pass row groups: TY / 4 rows per thread
+constexpr int SW_CR = 8;        // column-pass rows per thread
+constexpr int SW_RUN = 4;       // rows that share running window sums (FAST)
+constexpr int SW_PX = 4;        // row-pass pixels per thread
 
 struct SweepArgs {
     const float* ref;
@@ -51,14 +52,18 @@ struct SweepArgs {
     int W, H, N, P;
     int off;              // pixel-coordinate offset of the homography (1 = reference)
     int tiles_x, ntiles;
-    int ty;               // tile height (16 or 32)
-    int G;                // plane groups (aggregate mode): workgroups per tile
+    int tx, ty;           // tile shape (64 x 16 or 32 x 32)
+    int G;                // plane groups: workgroups per tile (and source, in a split reference sweep)
+    int S;                // reference mode: 1, or N workgroups per tile, one for each source
     float stdthresh, nccthresh, zfar;
     float* depth_out;     // reference mode
     int32_t* argmin;      // aggregate mode: written directly when G == 1 ...
     float* cmin;
     float* csec;
-    unsigned long long* top2;  // ... else every group's best two go to these per-pixel keys [2][H*W]
+    unsigned long long* top2;  // ... else every group's best two go to these per-pixel keys [2][H*W];
+                               // split reference sweep: best keys [N][H*W]
+    float* part;               // aggregate mode, small frames: each group's best cost, plane and second-best
+                               // cost instead, [3][G][H*W]
 };
 
 // The aggregated sweep's plane groups of one tile run in different
@@ -102,247 +107,355 @@ __device__ __forceinline__ void sweep_top2_insert(unsigned long long* top2, size
     if (offer != ~0ull) atomicMin(&top2[npix + i], offer);
 }
 
+// Waves per SIMD the register allocation aims at (1: as it comes).
+constexpr int sweep_waves(int R, bool FAST) { return FAST ? (R <= 4 ? 5 : 4) : 1; }
+
 template <bool FAST>
 __device__ inline float scale_mean(float s, float win, float rwin) {
     if constexpr (FAST) return s * rwin;
     else return s / win;
 }
 
-// One work item: plane group g of tile t (item = t * G + g).  Called by all
-// threads of a workgroup with the same item (it contains barriers).
-template <int R, int MODE, bool FAST, int TY = SW_TY>
-__device__ __forceinline__ void sweep_item(const SweepArgs& a, const int item) {
-    constexpr int TW = SW_TX + 2 * R;
-    constexpr int TH = TY + 2 * R;
-    constexpr int WIN = 2 * R + 1;
-    constexpr int NCG = SW_NCG;                 // column-pass row groups
-    constexpr int SW_CR = TY / SW_NCG;          // rows per thread in the column pass
-    constexpr int SW_PX = SW_TX * TY / SW_THREADS;  // pixels per thread in the row pass
-    constexpr int NCOL = NCG * TW;              // column-pass work items
-    constexpr int CV = SW_CR + 2 * R;           // column values per column item
-    constexpr int RV = SW_PX + 2 * R;           // row values per row item
-    static_assert(NCOL <= SW_THREADS, "window too large for the tile");
-    static_assert(TY % SW_NCG == 0 && (SW_TX * TY) % SW_THREADS == 0, "tile height");
-    __shared__ float sR[TH * TW];
-    __shared__ __align__(16) float sW[TH * TW];
-    __shared__ float sC[3][TY * TW];
+// The split reference sweep's key of a source's best NCC (> 0) and its plane:
+// the largest key is the largest NCC at its first plane, which is what the
+// strict-> scan over the planes keeps.  0: no NCC above 0.
+__device__ __forceinline__ unsigned long long best_key(float ncc, int plane) {
+    return ((unsigned long long)__float_as_uint(ncc) << 32) | (unsigned)~plane;
+}
 
-    const int t = item / a.G, g = item - (item / a.G) * a.G;
-    const int p0 = (g * a.P) / a.G, p1 = ((g + 1) * a.P) / a.G;
-    const int x0 = (t % a.tiles_x) * SW_TX;
+// The reference's NCC from the sums of the column means (kernels.cu:46-64,
+// :103-120), with its own roots and quotients.
+__device__ __forceinline__ float ncc_general(float m, float q, float pm, float win, float rmean, float rstd,
+                                             float stdthresh) {
+    m = m / win;
+    q = q / win;
+    pm = pm / win;
+    const float var = q - m * m;
+    const float sd = var > 0.f ? sqrtf(var) : 0.f;
+    if ((rstd < stdthresh) || (sd < stdthresh)) return 0.f;
+    return (pm - rmean * m) / (rstd * sd);
+}
+
+// The same bit for bit without the general root and division sequences,
+// where no operand is near the ends of the exponent range (zero sums, as in
+// windows without texture, take the general form too).
+template <int WIN>
+__device__ __forceinline__ float ncc_reference(float m0, float q0, float pm0, float rmean, float rstd,
+                                               float stdthresh) {
+    const float m = div_win<WIN>(m0), q = div_win<WIN>(q0), pm = div_win<WIN>(pm0);
+    const float var = q - m * m;
+    const float sd = sqrt_rn_gt1(var);    // its rounding test scales by powers of four
+    const float d = rstd * sd, x = pm - rmean * m;
+    const float mn = fminf(fminf(fabsf(m0), fabsf(pm0)), fminf(fminf(q0, var), fminf(d, fabsf(x))));
+    const float mx = fmaxf(fmaxf(fabsf(m0), fabsf(pm0)), fmaxf(fmaxf(q0, var), fmaxf(d, fabsf(x))));
+    float v = div_nr(x, d, rcp_nr(d));
+    if ((rstd < stdthresh) || (sd < stdthresh)) v = 0.f;
+    if (!(mn >= 0x1p-60f && mx <= 0x1p60f)) v = ncc_general(m0, q0, pm0, (float)WIN, rmean, rstd, stdthresh);
+    return v;
+}
+
+// One work item: plane group g of tile t (and of one source in a split
+// reference sweep).  Called by all threads of a workgroup with the same item
+// (it contains barriers).
+//
+// Bound by VALU issue, most of it the warp.  So:
+//   - 1024-pixel tiles warp 1.69 (64 x 16) or 1.56 (32 x 32) positions per
+//     pixel at a 9 x 9 window, where 32 x 16 tiles warped 1.88, and give the
+//     row pass 4 pixels per thread to run its sums along;
+//   - a thread warps position pairs of one column pair, RP rows apart, so the
+//     column terms of the homography are formed once per step;
+//   - whole steps whose tile lands inside the source need no bounds tests: a
+//     wave decides 64 steps at a time, one per lane, from the tile's corners;
+//   - reference order: the divisions by the window size and the projective
+//     divides are the short correctly rounded sequences of div_win and
+//     div_nr, with a check that falls back to '/'.
+// 640 x 480 x 8 x 256, 9 x 9, FAST: 1.57 ms, against 1.60 ms with 32 x 16
+// tiles.  637 x 479 x 4 x 199, 5 x 5, reference order: 1.06 ms against 2.37 ms
+// with one workgroup to a 32 x 16 tile and general divisions throughout.
+template <int R, int MODE, bool FAST, int TX, int TY>
+__device__ __forceinline__ void sweep_item(const SweepArgs& a, const int item) {
+    constexpr int TW = TX + 2 * R, TH = TY + 2 * R;
+    constexpr int LW = (TW + 3) / 4 * 4;           // LDS row stride: 16-byte row reads
+    constexpr int WIN = 2 * R + 1;
+    constexpr int NCOL = TY / SW_CR * TW;          // column-pass work items
+    constexpr int CV = SW_CR + 2 * R;              // column values per column item
+    constexpr int RV = (SW_PX + 2 * R + 3) / 4;    // float4 row values per row item
+    constexpr int PR = TW / 2, RP = SW_THREADS / PR, NP = (TH + RP - 1) / RP;  // warp: pairs per row, rows per pass
+    static_assert(NCOL <= SW_THREADS, "window too large for the tile");
+    static_assert(TW % 2 == 0 && TX * TY == SW_PX * SW_THREADS && TY % SW_CR == 0, "tile shape");
+    __shared__ __align__(16) float sW[TH * LW];
+    __shared__ __align__(16) float sC[3][TY * LW];
+    float* const sR = sW;                          // reference tile + halo, before the first warp
+
+    const int g = item % a.G;
+    const int ts = item / a.G, nS = MODE == 0 ? a.S : 1;
+    const int t = ts / nS;
+    const int s0 = nS > 1 ? ts - t * nS : 0, s1 = nS > 1 ? s0 + 1 : a.N;
+    const int p0 = (int)((long)g * a.P / a.G), p1 = (int)((long)(g + 1) * a.P / a.G);
+    const int x0 = (t % a.tiles_x) * TX;
     const int y0 = (t / a.tiles_x) * TY;
     const int tid = threadIdx.x;
     const int W = a.W, H = a.H;
-    const float win = (float)WIN, rwin = 1.f / (float)WIN;
+    const float offf = (float)a.off;
 
-    // Actual (reflected) image coordinate of each halo-tile position this
-    // thread warps; positions past W-1+R / H-1+R only feed discarded pixels.
-    // The reference-order sweep takes positions i = tid + k * threads; the
-    // fast one takes pairs (2q, 2q+1) of one row (TW is even), which share
-    // the homography's row terms.
-    constexpr int NWARP = (TH * TW + SW_THREADS - 1) / SW_THREADS;
-    constexpr int NPAIR = (TH * TW / 2 + SW_THREADS - 1) / SW_THREADS;
-    static_assert(TW % 2 == 0, "pairs of one row");
-    constexpr int NPOS = FAST ? 2 * NPAIR : NWARP;
-    int wgx[NPOS], wgy[NPOS];
+    // Positions this thread warps: column pair wc, rows wr + k RP; their
+    // (reflected) image coordinates.  Positions past W-1+R / H-1+R only feed
+    // discarded pixels.
+    const int wc = tid % PR, wr = tid / PR;
+    const bool warps = tid < PR * RP;
+    int gx[2];
+    float px[2], py[NP];
 #pragma unroll
-    for (int k = 0; k < NPOS; ++k) {
-        const int i = FAST ? 2 * (tid + (k / 2) * SW_THREADS) + (k & 1) : tid + k * SW_THREADS;
-        const int ty = i / TW, tx = i - (i / TW) * TW;
-        wgx[k] = reflect101(min(x0 - R + tx, W - 1 + R), W);
-        wgy[k] = reflect101(min(y0 - R + ty, H - 1 + R), H);
+    for (int e = 0; e < 2; ++e) {
+        gx[e] = reflect101(min(x0 - R + 2 * wc + e, W - 1 + R), W);
+        px[e] = (float)(gx[e] + a.off);
     }
 #pragma unroll
-    for (int k = 0; k < NPOS; ++k) {
-        const int i = FAST ? 2 * (tid + (k / 2) * SW_THREADS) + (k & 1) : tid + k * SW_THREADS;
-        if (i < TH * TW) sR[i] = a.ref[(size_t)wgy[k] * W + wgx[k]];
+    for (int k = 0; k < NP; ++k) {
+        const int row = wr + k * RP;
+        const int gy = reflect101(min(y0 - R + row, H - 1 + R), H);
+        py[k] = (float)(gy + a.off);
+        if (warps && row < TH) {
+#pragma unroll
+            for (int e = 0; e < 2; ++e) sR[row * LW + 2 * wc + e] = a.ref[(size_t)gy * W + gx[e]];
+        }
     }
     __syncthreads();
 
     // Column-pass item of this thread and its reference values (constant over
     // the whole sweep, so they live in registers).
     const bool col_active = tid < NCOL;
-    const int ccx = tid % TW, cg = min(tid / TW, NCG - 1);
+    const int ccx = tid % TW, cr = min(tid / TW, TY / SW_CR - 1) * SW_CR;
     float rv[CV];
 #pragma unroll
-    for (int i = 0; i < CV; ++i) rv[i] = sR[(cg * SW_CR + i) * TW + ccx];
-    // Row-pass pixels of this thread: (ox, oy), (ox+1, oy).
-    const int rox = SW_PX * (tid % (SW_TX / SW_PX));
-    const int roy = tid / (SW_TX / SW_PX);
+    for (int i = 0; i < CV; ++i) rv[i] = sR[(cr + i) * LW + ccx];
+    // Row-pass pixels of this thread: (rox .. rox + 3, roy).
+    const int rox = SW_PX * (tid % (TX / SW_PX));
+    const int roy = tid / (TX / SW_PX);
 
     // ---- reference window statistics (src/planesweep.cpp:108-119) ----
+    // (loops kept rolled: a small sweep spends its time fetching code)
+    const float win = (float)WIN, rwin = 1.f / (float)WIN;
     if (col_active) {
-#pragma unroll
+#pragma unroll 1
         for (int j = 0; j < SW_CR; ++j) {
-            float s1 = 0.f, s2 = 0.f;
+            float q1 = 0.f, q2 = 0.f;
 #pragma unroll
             for (int i = 0; i < WIN; ++i) {
-                s1 += rv[j + i];
-                s2 += rv[j + i] * rv[j + i];
+                const float r = sR[(cr + j + i) * LW + ccx];
+                q1 += r;
+                q2 += r * r;
             }
-            sC[0][(cg * SW_CR + j) * TW + ccx] = scale_mean<FAST>(s1, win, rwin);
-            sC[1][(cg * SW_CR + j) * TW + ccx] = scale_mean<FAST>(s2, win, rwin);
+            sC[0][(cr + j) * LW + ccx] = scale_mean<FAST>(q1, win, rwin);
+            sC[1][(cr + j) * LW + ccx] = scale_mean<FAST>(q2, win, rwin);
         }
     }
-    __syncthreads();
+    __syncthreads();   // sR's readers are done, too
+    static_assert(TX * TY <= TY * LW && TX * TY <= TH * LW, "the statistics fit sC[2] and sW");
+#pragma unroll 1
+    for (int k = 0; k < SW_PX; ++k) {
+        float m = 0.f, q = 0.f;
+#pragma unroll
+        for (int i = 0; i < WIN; ++i) {
+            m += sC[0][roy * LW + rox + k + i];
+            q += sC[1][roy * LW + rox + k + i];
+        }
+        m = scale_mean<FAST>(m, win, rwin);
+        q = scale_mean<FAST>(q, win, rwin);
+        const float var = q - m * m;
+        sC[2][SW_PX * tid + k] = m;
+        sW[SW_PX * tid + k] = var > 0.f ? sqrtf(var) : 0.f;
+    }
+    // read back by the thread that wrote them
     float rmean[SW_PX], rstd[SW_PX];
-    {
-        float c0[RV], c1[RV];
+    bool textured[SW_PX];
 #pragma unroll
-        for (int i = 0; i < RV; ++i) {
-            c0[i] = sC[0][roy * TW + rox + i];
-            c1[i] = sC[1][roy * TW + rox + i];
-        }
-#pragma unroll
-        for (int k = 0; k < SW_PX; ++k) {
-            float m = 0.f, q = 0.f;
-#pragma unroll
-            for (int i = 0; i < WIN; ++i) {
-                m += c0[k + i];
-                q += c1[k + i];
-            }
-            m = scale_mean<FAST>(m, win, rwin);
-            q = scale_mean<FAST>(q, win, rwin);
-            const float var = q - m * m;
-            rmean[k] = m;
-            rstd[k] = var > 0.f ? sqrtf(var) : 0.f;
-        }
+    for (int k = 0; k < SW_PX; ++k) {
+        rmean[k] = sC[2][SW_PX * tid + k];
+        rstd[k] = sW[SW_PX * tid + k];
+        textured[k] = !(rstd[k] < a.stdthresh);
     }
     __syncthreads();
 
+    // Steps [first, first + 64) whose tile, halo included, lands inside the
+    // source with a margin: the tile's image is the convex quadrilateral of
+    // its corners' images while the projective divisor keeps its sign.  The
+    // margin covers the rounding of the positions; the divisor's range keeps
+    // the quotients' operands in div_nr's.  Uniform over the workgroup.
+    const int nstep = (p1 - p0) * (s1 - s0);
+    const bool small = (size_t)W * H < (1u << 30) && W < (1 << 22);   // byte offsets of inside samples
+    auto inside_steps = [&](int first) -> unsigned long long {
+        const int st = first + (int)(tid & 63);
+        bool in = false;
+        if (nstep >= 8 && st < nstep && small) {   // not worth its latency for a few steps
+            const int s = MODE == 0 ? s0 + st / (p1 - p0) : st % a.N;
+            const int p = p0 + (MODE == 0 ? st % (p1 - p0) : st / a.N);
+            const float* __restrict__ h = a.Hs + ((size_t)s * a.P + p) * 9;
+            const float ex = 0.0625f + 0x1p-18f * (float)W, ey = 0.0625f + 0x1p-18f * (float)H;
+            in = true;
+#pragma unroll 1
+            for (int c = 0; c < 4; ++c) {
+                const float cx = (float)((c & 1 ? min(x0 + TX + R - 1, W - 1) : max(x0 - R, 0)) + a.off);
+                const float cy = (float)((c & 2 ? min(y0 + TY + R - 1, H - 1) : max(y0 - R, 0)) + a.off);
+                const float vz = h[6] * cx + h[7] * cy + h[8];
+                const float x = (h[0] * cx + h[1] * cy + h[2]) / vz - offf;
+                const float y = (h[3] * cx + h[4] * cy + h[5]) / vz - offf;
+                in = in && vz >= 0x1p-20f && vz <= 0x1p20f && x >= ex && x <= (float)(W - 1) - ex && y >= ey &&
+                     y <= (float)(H - 1) - ey;
+            }
+        }
+        return __ballot(in);
+    };
+
     // One (plane, source) step: warp into sW, window sums, NCC of my pixels.
-    auto plane_ncc = [&](const float* __restrict__ src, const float* __restrict__ Hm, float ncc[SW_PX]) {
+    auto plane_ncc = [&](const float* __restrict__ src, const float* __restrict__ Hm, bool inside, float (&ncc)[SW_PX]) {
         const float h0 = Hm[0], h1 = Hm[1], h2 = Hm[2], h3 = Hm[3], h4 = Hm[4], h5 = Hm[5], h6 = Hm[6],
                     h7 = Hm[7], h8 = Hm[8];
-        const float offf = (float)a.off;
-        if constexpr (FAST) {
+        auto warp = [&](auto in) {
+            constexpr bool IN = decltype(in)::value;
+            float cx[2], cy[2], cz[2];   // column terms
 #pragma unroll
-            for (int k = 0; k < NPAIR; ++k) {
-                const int q = tid + k * SW_THREADS;
-                if (q < TH * TW / 2) {
-                    // explicit fused multiply-adds (no contraction left to the
-                    // compiler), so every kernel that inlines this computes
-                    // the same bits; the row terms are the pair's
-                    const float py = (float)(wgy[2 * k] + a.off);
-                    const float cx = __builtin_fmaf(h1, py, h2), cy = __builtin_fmaf(h4, py, h5),
-                                cz = __builtin_fmaf(h7, py, h8);
-                    float out[2];
+            for (int e = 0; e < 2; ++e) {
+                cx[e] = h0 * px[e];
+                cy[e] = h3 * px[e];
+                cz[e] = h6 * px[e];
+            }
 #pragma unroll
-                    for (int e = 0; e < 2; ++e) {
-                        const float px = (float)(wgx[2 * k + e] + a.off);
-                        const float vx = __builtin_fmaf(h0, px, cx);
-                        const float vy = __builtin_fmaf(h3, px, cy);
-                        const float vz = __builtin_fmaf(h6, px, cz);
+            for (int k = 0; k < NP; ++k) {
+                if (k == NP - 1 && wr + k * RP >= TH) break;
+                float out[2];
+                // FAST: the row terms are the pair's
+                const float fx = __builtin_fmaf(h1, py[k], h2), fy = __builtin_fmaf(h4, py[k], h5),
+                            fz = __builtin_fmaf(h7, py[k], h8);
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    if constexpr (FAST) {
+                        const float vx = __builtin_fmaf(h0, px[e], fx);
+                        const float vy = __builtin_fmaf(h3, px[e], fy);
+                        const float vz = __builtin_fmaf(h6, px[e], fz);
                         const float rz = __builtin_amdgcn_rcpf(vz);
-                        out[e] = bilinear_sample_fma(src, W, H, __builtin_fmaf(vx, rz, -offf),
-                                                     __builtin_fmaf(vy, rz, -offf));
+                        const float x = __builtin_fmaf(vx, rz, -offf), y = __builtin_fmaf(vy, rz, -offf);
+                        out[e] = bilinear_sample_fma<!IN>(src, W, H, x, y);
+                    } else {
+                        const float vx = (cx[e] + h1 * py[k]) + h2;
+                        const float vy = (cy[e] + h4 * py[k]) + h5;
+                        const float vz = (cz[e] + h7 * py[k]) + h8;
+                        if constexpr (IN) {
+                            const float rz = rcp_nr(vz);
+                            out[e] = bilinear_inside(src, W, div_nr(vx, vz, rz) - offf, div_nr(vy, vz, rz) - offf);
+                        } else {
+                            out[e] = bilinear_sample(src, W, H, vx / vz - offf, vy / vz - offf);
+                        }
                     }
-                    *reinterpret_cast<float2*>(&sW[2 * q]) = make_float2(out[0], out[1]);
                 }
+                *reinterpret_cast<float2*>(&sW[(wr + k * RP) * LW + 2 * wc]) = make_float2(out[0], out[1]);
             }
-        } else {
-#pragma unroll
-            for (int k = 0; k < NWARP; ++k) {
-                const int i = tid + k * SW_THREADS;
-                if (i < TH * TW) {
-                    const float px = (float)(wgx[k] + a.off), py = (float)(wgy[k] + a.off);
-                    const float vx = dot3(h0, h1, h2, px, py, 1.f);
-                    const float vy = dot3(h3, h4, h5, px, py, 1.f);
-                    const float vz = dot3(h6, h7, h8, px, py, 1.f);
-                    sW[i] = bilinear_sample(src, W, H, vx / vz - offf, vy / vz - offf);
-                }
-            }
+        };
+        if (warps) {
+            if (inside) warp(std::true_type{});
+            else warp(std::false_type{});
         }
         __syncthreads();
         if (col_active) {
             float wv[CV];
 #pragma unroll
-            for (int i = 0; i < CV; ++i) wv[i] = sW[(cg * SW_CR + i) * TW + ccx];
+            for (int i = 0; i < CV; ++i) wv[i] = sW[(cr + i) * LW + ccx];
+            float* const c0 = &sC[0][cr * LW + ccx];
+            float* const c1 = &sC[1][cr * LW + ccx];
+            float* const c2 = &sC[2][cr * LW + ccx];
             if constexpr (FAST) {
-                // running window sums down the column
-                float s1 = 0.f, s2 = 0.f, s3 = 0.f;
-#pragma unroll
-                for (int i = 0; i < WIN; ++i) {
-                    s1 += wv[i];
-                    s2 = __builtin_fmaf(wv[i], wv[i], s2);
-                    s3 = __builtin_fmaf(rv[i], wv[i], s3);
-                }
+                // window sums, running down groups of four rows
+                float q1 = 0.f, q2 = 0.f, q3 = 0.f;
 #pragma unroll
                 for (int j = 0; j < SW_CR; ++j) {
-                    if (j > 0) {
+                    if (j % SW_RUN == 0) {
+                        q1 = q2 = q3 = 0.f;
+#pragma unroll
+                        for (int i = 0; i < WIN; ++i) {
+                            const float w = wv[j + i];
+                            q1 += w;
+                            q2 = __builtin_fmaf(w, w, q2);
+                            q3 = __builtin_fmaf(rv[j + i], w, q3);
+                        }
+                    } else {
                         const float wa = wv[j + 2 * R], wd = wv[j - 1];
-                        s1 += wa - wd;
-                        s2 = __builtin_fmaf(wa, wa, __builtin_fmaf(-wd, wd, s2));
-                        s3 = __builtin_fmaf(rv[j + 2 * R], wa, __builtin_fmaf(-rv[j - 1], wd, s3));
+                        q1 += wa - wd;
+                        q2 = __builtin_fmaf(wa, wa, __builtin_fmaf(-wd, wd, q2));
+                        q3 = __builtin_fmaf(rv[j + 2 * R], wa, __builtin_fmaf(-rv[j - 1], wd, q3));
                     }
-                    sC[0][(cg * SW_CR + j) * TW + ccx] = s1 * rwin;
-                    sC[1][(cg * SW_CR + j) * TW + ccx] = s2 * rwin;
-                    sC[2][(cg * SW_CR + j) * TW + ccx] = s3 * rwin;
+                    c0[j * LW] = q1 * rwin;
+                    c1[j * LW] = q2 * rwin;
+                    c2[j * LW] = q3 * rwin;
                 }
             } else {
-#pragma unroll
-                for (int j = 0; j < SW_CR; ++j) {
-                    float s1 = 0.f, s2 = 0.f, s3 = 0.f;
+                auto sums = [&](int j, float& q1, float& q2, float& q3) {
+                    q1 = q2 = q3 = 0.f;
 #pragma unroll
                     for (int i = 0; i < WIN; ++i) {
                         const float w = wv[j + i];
-                        s1 += w;
-                        s2 += w * w;
-                        s3 += rv[j + i] * w;
+                        q1 += w;
+                        q2 += w * w;
+                        q3 += rv[j + i] * w;
                     }
-                    sC[0][(cg * SW_CR + j) * TW + ccx] = s1 / win;
-                    sC[1][(cg * SW_CR + j) * TW + ccx] = s2 / win;
-                    sC[2][(cg * SW_CR + j) * TW + ccx] = s3 / win;
+                };
+                float mn = __builtin_inff(), mx = 0.f;
+#pragma unroll
+                for (int j = 0; j < SW_CR; ++j) {
+                    float q1, q2, q3;
+                    sums(j, q1, q2, q3);
+                    mn = fminf(mn, fminf(fminf(fabsf(q1), q2), fabsf(q3)));
+                    mx = fmaxf(mx, fmaxf(fmaxf(fabsf(q1), q2), fabsf(q3)));
+                    c0[j * LW] = div_win<WIN>(q1);
+                    c1[j * LW] = div_win<WIN>(q2);
+                    c2[j * LW] = div_win<WIN>(q3);
+                }
+                if (!(mn >= 0x1p-60f && mx <= 0x1p60f)) {
+#pragma unroll
+                    for (int j = 0; j < SW_CR; ++j) {
+                        float q1, q2, q3;
+                        sums(j, q1, q2, q3);
+                        c0[j * LW] = q1 / win;
+                        c1[j * LW] = q2 / win;
+                        c2[j * LW] = q3 / win;
+                    }
                 }
             }
         }
         __syncthreads();
-        float c0[RV], c1[RV], c2[RV];
+        // sums of the row windows, one of the three quantities at a time
+        float sum[3][SW_PX];
 #pragma unroll
-        for (int i = 0; i < RV; ++i) {
-            c0[i] = sC[0][roy * TW + rox + i];
-            c1[i] = sC[1][roy * TW + rox + i];
-            c2[i] = sC[2][roy * TW + rox + i];
-        }
-        if constexpr (FAST) {
-            float m = 0.f, q = 0.f, pm = 0.f;
+        for (int q = 0; q < 3; ++q) {
+            float v[4 * RV];
+#pragma unroll
+            for (int i = 0; i < RV; ++i) {
+                const f32x4 f = *reinterpret_cast<const f32x4*>(&sC[q][roy * LW + rox + 4 * i]);
+                v[4 * i] = f.x; v[4 * i + 1] = f.y; v[4 * i + 2] = f.z; v[4 * i + 3] = f.w;
+            }
+            float m = 0.f;
 #pragma unroll
             for (int k = 0; k < SW_PX; ++k) {
-                if (k == 0) {
+                if (!FAST || k % 2 == 0) {
+                    m = 0.f;
 #pragma unroll
-                    for (int i = 0; i < WIN; ++i) {
-                        m += c0[i];
-                        q += c1[i];
-                        pm += c2[i];
-                    }
+                    for (int i = 0; i < WIN; ++i) m += v[k + i];
                 } else {
-                    m += c0[k + 2 * R] - c0[k - 1];
-                    q += c1[k + 2 * R] - c1[k - 1];
-                    pm += c2[k + 2 * R] - c2[k - 1];
+                    m += v[k + 2 * R] - v[k - 1];
                 }
+                sum[q][k] = m;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < SW_PX; ++k) {
+            const float m = sum[0][k], q = sum[1][k], pm = sum[2][k];
+            if constexpr (FAST) {
                 const float mm = m * rwin, qq = q * rwin, pp = pm * rwin;
                 const float var = __builtin_fmaf(-mm, mm, qq);
                 const float sd = var > 0.f ? __builtin_amdgcn_sqrtf(var) : 0.f;
-                if ((rstd[k] < a.stdthresh) || (sd < a.stdthresh)) ncc[k] = 0.f;
-                else ncc[k] = __builtin_fmaf(-rmean[k], mm, pp) * __builtin_amdgcn_rcpf(rstd[k] * sd);
-            }
-        } else {
-#pragma unroll
-            for (int k = 0; k < SW_PX; ++k) {
-                float m = 0.f, q = 0.f, pm = 0.f;
-#pragma unroll
-                for (int i = 0; i < WIN; ++i) {
-                    m += c0[k + i];
-                    q += c1[k + i];
-                    pm += c2[k + i];
-                }
-                m = m / win;
-                q = q / win;
-                pm = pm / win;
-                const float var = q - m * m;
-                const float sd = var > 0.f ? sqrtf(var) : 0.f;
-                if ((rstd[k] < a.stdthresh) || (sd < a.stdthresh)) ncc[k] = 0.f;
-                else ncc[k] = (pm - rmean[k] * m) / (rstd[k] * sd);
+                const float v = __builtin_fmaf(-rmean[k], mm, pp) * __builtin_amdgcn_rcpf(rstd[k] * sd);
+                ncc[k] = textured[k] && !(sd < a.stdthresh) ? v : 0.f;
+            } else {
+                ncc[k] = ncc_reference<WIN>(m, q, pm, rmean[k], rstd[k], a.stdthresh);
             }
         }
         // No barrier here: the next warp writes sW (its readers passed the
@@ -351,34 +464,76 @@ __device__ __forceinline__ void sweep_item(const SweepArgs& a, const int item) {
     };
 
     const size_t npix = (size_t)W * H;
+    const int x = x0 + rox, y = y0 + roy;
+    // Results that go to per-pixel keys change hands through LDS, so that a
+    // wave's atomics cover runs of neighbouring pixels: thread t takes pixels
+    // t + 256 k of the tile (with four consecutive pixels per lane the same
+    // the sweep of 563 x 317 x 8 x 48, 3 x 3, took 466 us instead of 214).
+    float* const xch = sC[0];
+    static_assert(3 * TX * TY <= 3 * TY * LW, "the exchange fits sC");
+    const int mine = roy * TX + rox;
+    auto put = [&](int f, int k, float v) { xch[f * TX * TY + mine + k] = v; };
+    auto got = [&](int f, int k) { return xch[f * TX * TY + tid + k * SW_THREADS]; };
+    auto pixel = [&](int k, size_t& i) {   // of my k-th exchanged pixel; false outside the image
+        const int e = tid + k * SW_THREADS, ex = x0 + e % TX, ey = y0 + e / TX;
+        i = (size_t)ey * W + ex;
+        return ex < W && ey < H;
+    };
+    unsigned long long in = 0;
+    int step = 0;
+    auto next_inside = [&]() {   // of step `step`, then the next one
+        if ((step & 63) == 0) in = inside_steps(step);
+        return ((in >> (step++ & 63)) & 1) != 0;
+    };
     if constexpr (MODE == 0) {
         float gsum[SW_PX], gcnt[SW_PX];
 #pragma unroll
         for (int k = 0; k < SW_PX; ++k) { gsum[k] = 0.f; gcnt[k] = 0.f; }
-        for (int s = 0; s < a.N; ++s) {
+        for (int s = s0; s < s1; ++s) {
             const float* src = a.src + (size_t)s * npix;
-            float best[SW_PX], bd[SW_PX];
+            float best[SW_PX];
+            int bp[SW_PX];
 #pragma unroll
-            for (int k = 0; k < SW_PX; ++k) { best[k] = 0.f; bd[k] = 0.f; }
-            for (int p = 0; p < a.P; ++p) {
+            for (int k = 0; k < SW_PX; ++k) { best[k] = 0.f; bp[k] = -1; }
+            for (int p = p0; p < p1; ++p) {
                 float ncc[SW_PX];
-                plane_ncc(src, a.Hs + ((size_t)s * a.P + p) * 9, ncc);
-                const float d = a.depths[p];
+                plane_ncc(src, a.Hs + ((size_t)s * a.P + p) * 9, next_inside(), ncc);
 #pragma unroll
                 for (int k = 0; k < SW_PX; ++k)
-                    if (ncc[k] > best[k]) { best[k] = ncc[k]; bd[k] = d; }
+                    if (ncc[k] > best[k]) { best[k] = ncc[k]; bp[k] = p; }
             }
+            if (a.top2) {
+                __syncthreads();
 #pragma unroll
-            for (int k = 0; k < SW_PX; ++k)
-                if (best[k] > a.nccthresh) { gsum[k] += bd[k]; gcnt[k] += 1.f; }
+                for (int k = 0; k < SW_PX; ++k) {
+                    put(0, k, best[k]);
+                    put(1, k, __int_as_float(bp[k]));
+                }
+                __syncthreads();
+#pragma unroll
+                for (int k = 0; k < SW_PX; ++k) {
+                    size_t i;
+                    const int p = __float_as_int(got(1, k));
+                    if (pixel(k, i) && p >= 0) atomicMax(&a.top2[(size_t)s * npix + i], best_key(got(0, k), p));
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < SW_PX; ++k) {
+                    if (best[k] > a.nccthresh) {
+                        gsum[k] += bp[k] >= 0 ? a.depths[bp[k]] : 0.f;
+                        gcnt[k] += 1.f;
+                    }
+                }
+            }
         }
+        if (!a.top2) {
 #pragma unroll
-        for (int k = 0; k < SW_PX; ++k) {
-            const int x = x0 + rox + k, y = y0 + roy;
-            if (x < W && y < H) {
-                float v = (gcnt[k] != 0.f) ? gsum[k] / gcnt[k] : __builtin_nanf("");
-                if (v != v) v = a.zfar;
-                a.depth_out[(size_t)y * W + x] = v;
+            for (int k = 0; k < SW_PX; ++k) {
+                if (x + k < W && y < H) {
+                    float v = (gcnt[k] != 0.f) ? gsum[k] / gcnt[k] : __builtin_nanf("");
+                    if (v != v) v = a.zfar;
+                    a.depth_out[(size_t)y * W + x + k] = v;
+                }
             }
         }
     } else {
@@ -388,57 +543,73 @@ __device__ __forceinline__ void sweep_item(const SweepArgs& a, const int item) {
 #pragma unroll
         for (int k = 0; k < SW_PX; ++k) { cmin[k] = inf; csec[k] = inf; arg[k] = -1; }
         const float fN = (float)a.N;
+        const bool exact = FAST && (a.N & (a.N - 1)) == 0;   // a product with 1 / N is the quotient
         for (int p = p0; p < p1; ++p) {
             float acc[SW_PX];
 #pragma unroll
             for (int k = 0; k < SW_PX; ++k) acc[k] = 0.f;
             for (int s = 0; s < a.N; ++s) {
                 float ncc[SW_PX];
-                plane_ncc(a.src + (size_t)s * npix, a.Hs + ((size_t)s * a.P + p) * 9, ncc);
+                plane_ncc(a.src + (size_t)s * npix, a.Hs + ((size_t)s * a.P + p) * 9, next_inside(), ncc);
 #pragma unroll
                 for (int k = 0; k < SW_PX; ++k) acc[k] += ncc[k];
             }
 #pragma unroll
             for (int k = 0; k < SW_PX; ++k) {
-                const float c = -acc[k] / fN;
+                const float c = exact ? -acc[k] * (1.f / fN) : -acc[k] / fN;
                 if (c < cmin[k]) { csec[k] = cmin[k]; cmin[k] = c; arg[k] = p; }
                 else if (c < csec[k]) csec[k] = c;
             }
         }
+        __syncthreads();
 #pragma unroll
         for (int k = 0; k < SW_PX; ++k) {
-            const int x = x0 + rox + k, y = y0 + roy;
-            if (x < W && y < H) {
-                const size_t i = (size_t)y * W + x;
-                if (a.G > 1) {
-                    sweep_top2_insert(a.top2, npix, i, cmin[k], arg[k], csec[k]);
-                } else {
-                    a.argmin[i] = arg[k];
-                    a.cmin[i] = cmin[k];
-                    a.csec[i] = csec[k];
-                }
+            put(0, k, cmin[k]);
+            put(1, k, __int_as_float(arg[k]));
+            put(2, k, csec[k]);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < SW_PX; ++k) {
+            size_t i;
+            if (!pixel(k, i)) continue;
+            const float c1 = got(0, k), c2 = got(2, k);
+            const int p = __float_as_int(got(1, k));
+            if (a.G > 1 && a.part) {
+                float* const o = a.part + (size_t)g * npix + i;
+                const size_t plane = (size_t)a.G * npix;
+                o[0] = c1;
+                o[plane] = __int_as_float(p);
+                o[2 * plane] = c2;
+            } else if (a.G > 1) {
+                sweep_top2_insert(a.top2, npix, i, c1, p, c2);
+            } else {
+                a.argmin[i] = p;
+                a.cmin[i] = c1;
+                a.csec[i] = c2;
             }
         }
     }
 }
 
-// The fast variant is held to 72 VGPRs (7 waves per SIMD instead of 6;
-// measured 1.73 against 1.76 ms at 640x480 x 8 x 256, 9x9: two registers
-// spill; at 8 waves sixteen do and it is slower).
-template <int R, int MODE, bool FAST, int TY>
-__global__ __launch_bounds__(SW_THREADS) __attribute__((amdgpu_waves_per_eu(FAST ? 7 : 1))) void sweep_fused_kernel(SweepArgs a) {
-    if ((int)blockIdx.x >= a.ntiles * a.G) return;
-    sweep_item<R, MODE, FAST, TY>(a, xcd_tile(blockIdx.x, a.ntiles * a.G));
+// The fast variant is held to 5 waves per SIMD (640 x 480 x 8 x 256, 9 x 9:
+// 1.56 ms, as with 6, which spills; 4 took 1.62); windows above 9 x 9 need up
+// to 128 VGPRs.
+template <int R, int MODE, bool FAST, int TX, int TY>
+__global__ __launch_bounds__(SW_THREADS) __attribute__((amdgpu_waves_per_eu(sweep_waves(R, FAST)))) void sweep_fused_kernel(SweepArgs a) {
+    const int nitems = a.ntiles * a.G * a.S;
+    if ((int)blockIdx.x >= nitems) return;
+    sweep_item<R, MODE, FAST, TX, TY>(a, xcd_tile(blockIdx.x, nitems));
 }
 
 // Many frames (uneven sizes, plane and source counts) in one persistent
 // launch: workgroups take items from a device counter until all frames'
 // items are done.  Item g belongs to the frame f with off[f] <= g < off[f+1].
 // Every item is computed exactly as in sweep_fused_kernel.
-template <int R, int MODE, bool FAST, int TY>
-__global__ __launch_bounds__(SW_THREADS) void sweep_batch_kernel(const SweepArgs* __restrict__ frames,
-                                                                 const int* __restrict__ off, int nframes, int total,
-                                                                 unsigned* __restrict__ counter) {
+template <int R, int MODE, bool FAST, int TX, int TY>
+__global__ __launch_bounds__(SW_THREADS) __attribute__((amdgpu_waves_per_eu(sweep_waves(R, FAST))))
+void sweep_batch_kernel(const SweepArgs* __restrict__ frames, const int* __restrict__ off, int nframes, int total,
+                        unsigned* __restrict__ counter) {
     __shared__ int s_item;
     for (;;) {
         if (threadIdx.x == 0) s_item = (int)atomicAdd(counter, 1u);
@@ -453,8 +624,28 @@ __global__ __launch_bounds__(SW_THREADS) void sweep_batch_kernel(const SweepArgs
             else hi = mid - 1;
         }
         const SweepArgs a = frames[lo];
-        sweep_item<R, MODE, FAST, TY>(a, gi - off[lo]);
+        sweep_item<R, MODE, FAST, TX, TY>(a, gi - off[lo]);
     }
+}
+
+// The split reference sweep's depth from the sources' best keys, in the
+// order and arithmetic of sweep_item's own reduction.
+__global__ void sweep_best_depth_kernel(const unsigned long long* __restrict__ best, size_t npix, int N,
+                                        const float* __restrict__ depths, float nccthresh, float zfar,
+                                        float* __restrict__ out) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= npix) return;
+    float sum = 0.f, cnt = 0.f;
+    for (int s = 0; s < N; ++s) {
+        const unsigned long long k = best[(size_t)s * npix + i];
+        if (__uint_as_float((unsigned)(k >> 32)) > nccthresh) {
+            sum += k ? depths[~(unsigned)k] : 0.f;
+            cnt += 1.f;
+        }
+    }
+    float v = cnt != 0.f ? sum / cnt : __builtin_nanf("");
+    if (v != v) v = zfar;
+    out[i] = v;
 }
 
 // The outputs from the per-pixel keys of the plane groups (all-ones: no
@@ -468,6 +659,60 @@ __global__ void sweep_top2_kernel(const unsigned long long* __restrict__ top2, s
     arg[i] = k0 == ~0ull ? -1 : (int32_t)(unsigned)k0;
     cmin[i] = k0 == ~0ull ? inf : sweep_key_cost(k0);
     csec[i] = k1 == ~0ull ? inf : sweep_key_cost(k1);
+}
+
+// Folds the best cost a1 at plane ap and second-best a2 of later planes into
+// c1, p1, c2, as the scan over all planes does.
+__device__ __forceinline__ void merge_bests(float a1, int ap, float a2, float& c1, int& p1, float& c2) {
+    if (a1 < c1) {
+        c2 = a2 < c1 ? a2 : c1;
+        c1 = a1;
+        p1 = ap;
+    } else if (a1 < c2) {
+        c2 = a1;
+    }
+}
+
+// The outputs from the plane groups' own bests (-0 folded into +0, as in the
+// keys).  A wave takes 64 pixels, the four waves of a workgroup a quarter of
+// the groups each, eight loads of each array in flight: with one thread to a
+// pixel's groups the loads of a small frame were one long chain.
+__global__ __launch_bounds__(256) void sweep_merge_kernel(const float* __restrict__ part, size_t npix, int G,
+                                                          int32_t* __restrict__ arg, float* __restrict__ cmin,
+                                                          float* __restrict__ csec) {
+    __shared__ float s1[4][64], s2[4][64];
+    __shared__ int sp[4][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const size_t i = (size_t)blockIdx.x * 64 + lane, plane = (size_t)G * npix;
+    float c1 = __builtin_inff(), c2 = c1;
+    int p1 = -1;
+    if (i < npix) {
+        const int g1 = (w + 1) * G / 4;
+        for (int g = w * G / 4; g < g1; g += 8) {
+            float a1[8], a2[8];
+            int ap[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const float* const o = part + (size_t)min(g + k, g1 - 1) * npix + i;
+                a1[k] = o[0];
+                ap[k] = __float_as_int(o[plane]);
+                a2[k] = o[2 * plane];
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (g + k < g1) merge_bests(a1[k], ap[k], a2[k], c1, p1, c2);
+        }
+    }
+    s1[w][lane] = c1;
+    sp[w][lane] = p1;
+    s2[w][lane] = c2;
+    __syncthreads();
+    if (w != 0 || i >= npix) return;
+#pragma unroll
+    for (int k = 1; k < 4; ++k) merge_bests(s1[k][lane], sp[k][lane], s2[k][lane], c1, p1, c2);
+    arg[i] = p1;
+    cmin[i] = c1 + 0.0f;
+    csec[i] = c2 + 0.0f;
 }
 
 // ---- FP64 homographies -----------------------------------------------------
@@ -554,16 +799,17 @@ static void d_relative(const float* Rref, const float* tref, const float* Rsrc, 
 
 template <int R>
 static int launch_sweep_r(const SweepArgs& a, int mode, bool fast, hipStream_t st) {
-    const dim3 grid((unsigned)(a.ntiles * a.G)), block(SW_THREADS);
+    const dim3 grid((unsigned)(a.ntiles * a.G * a.S)), block(SW_THREADS);
+    const bool tall = a.ty == 32;
     if (mode == 0) {
-        if (fast) sweep_fused_kernel<R, 0, true, 16><<<grid, block, 0, st>>>(a);
-        else sweep_fused_kernel<R, 0, false, 16><<<grid, block, 0, st>>>(a);
-    } else if (a.ty == 32) {
-        if (fast) sweep_fused_kernel<R, 1, true, 32><<<grid, block, 0, st>>>(a);
-        else sweep_fused_kernel<R, 1, false, 32><<<grid, block, 0, st>>>(a);
+        if (tall) sweep_fused_kernel<R, 0, false, 32, 32><<<grid, block, 0, st>>>(a);
+        else sweep_fused_kernel<R, 0, false, 64, 16><<<grid, block, 0, st>>>(a);
+    } else if (tall) {
+        if (fast) sweep_fused_kernel<R, 1, true, 32, 32><<<grid, block, 0, st>>>(a);
+        else sweep_fused_kernel<R, 1, false, 32, 32><<<grid, block, 0, st>>>(a);
     } else {
-        if (fast) sweep_fused_kernel<R, 1, true, 16><<<grid, block, 0, st>>>(a);
-        else sweep_fused_kernel<R, 1, false, 16><<<grid, block, 0, st>>>(a);
+        if (fast) sweep_fused_kernel<R, 1, true, 64, 16><<<grid, block, 0, st>>>(a);
+        else sweep_fused_kernel<R, 1, false, 64, 16><<<grid, block, 0, st>>>(a);
     }
     return launch_status("sweep_fused_kernel");
 }
@@ -584,27 +830,42 @@ static int launch_sweep(SweepArgs a, int winsize, int mode, bool fast, hipStream
     }
 }
 
-// Tiles of the image, and plane groups per tile so that a launch has enough
-// workgroups to keep 256 CUs busy to the end (about 14400 at 32 x 16 tiles:
-// 24 groups of the 600 tiles of a 640 x 480 frame, measured the fastest of
-// 1..64 groups).  PSW_SWEEP_GROUPS overrides the choice.
-constexpr long SW_TARGET_ITEMS = 14400;
-// The aggregated sweep's tile height: PSW_SWEEP_TY (16 or 32) or 16.
+// Tiles of the image, and plane groups per tile: enough workgroups to keep
+// 256 CUs busy to the end, with enough (plane, source) steps each to be worth
+// the reference statistics and the merge (9; 6 where a larger window makes a
+// step longer; or one workgroup per CU, where that takes more), and whole
+// rounds of resident workgroups (SW_SLOTS: five per CU) where there are few.
+// Measured over 30 sizes from 112 x 88 to 981 x 553 (1.36 times as fast on
+// average as 32 x 16 tiles with 14400 workgroups): 6, 9 and 12 steps are
+// within 3 % of each other on average, and with 9 / 6 no size is slower by
+// more than 3 %.
+// PSW_SWEEP_GROUPS overrides the choice (up to 64).
+constexpr long SW_TARGET_ITEMS = 5120, SW_SLOTS = 1280;
+// The tile shape: PSW_SWEEP_TY 16 (64 x 16) or 32 (32 x 32), else 0 for the
+// one that covers the frames with fewer tiles.  Results do not depend on it.
 static int sweep_tile_height() {
     const char* e = getenv("PSW_SWEEP_TY");
-    return (e && atoi(e) == 32) ? 32 : 16;
+    const int v = e ? atoi(e) : 0;
+    return v == 16 || v == 32 ? v : 0;
+}
+static long sweep_tiles(int W, int H, int ty) {
+    const int tx = ty == 32 ? 32 : 64;
+    return (long)((W + tx - 1) / tx) * ((H + ty - 1) / ty);
 }
 
-static void sweep_layout(SweepArgs& a, bool allow_groups, int ty = SW_TY) {
-    a.ty = ty;
-    a.tiles_x = (a.W + SW_TX - 1) / SW_TX;
-    const int tiles_y = (a.H + a.ty - 1) / a.ty;
-    a.ntiles = a.tiles_x * tiles_y;
+static void sweep_layout(SweepArgs& a, bool allow_groups, int ty, int winsize) {
+    a.ty = ty ? ty : sweep_tiles(a.W, a.H, 32) < sweep_tiles(a.W, a.H, 16) ? 32 : 16;
+    a.tx = a.ty == 32 ? 32 : 64;
+    a.tiles_x = (a.W + a.tx - 1) / a.tx;
+    a.ntiles = (int)sweep_tiles(a.W, a.H, a.ty);
     a.G = 1;
+    a.S = 1;
     if (!allow_groups) return;
-    int G = (int)((SW_TARGET_ITEMS * 16 / a.ty + a.ntiles / 2) / a.ntiles);
-    if (const char* e = getenv("PSW_SWEEP_GROUPS")) G = atoi(e);
-    a.G = std::max(1, std::min(G, std::min(a.P, 64)));
+    const long nt = a.ntiles;
+    long G = std::min((SW_TARGET_ITEMS + nt / 2) / nt, std::max((long)a.N * a.P / (winsize > 9 ? 6 : 9), 256 / nt));
+    if (nt * G > SW_SLOTS && nt * G < 3 * SW_SLOTS) G = nt * G / SW_SLOTS * SW_SLOTS / nt;
+    if (const char* e = getenv("PSW_SWEEP_GROUPS")) G = std::min(atoi(e), 64);
+    a.G = (int)std::max(1L, std::min(G, (long)std::min(a.P, 128)));
 }
 
 static int check_sweep_args(const float* d_ref, const float* d_src, int width, int height, int nsrc,
@@ -653,20 +914,38 @@ static int scratch_address(void** out) {
     return PSW_OK;
 }
 
-// The aggregated sweep's launch and, with plane groups, the per-pixel keys
-// in `ws` (SW_KEY_BYTES per pixel: cleared first, turned into the outputs
-// after).
+// The aggregated sweep's launch and, with plane groups, their workspace `ws`
+// of sweep_ws_bytes: the groups' own bests, merged after, where those fit
+// SW_PART_BYTES (frames up to 320 x 240 at the default group count); else the
+// per-pixel keys (SW_KEY_BYTES per pixel: cleared first, turned into the
+// outputs after).  Small frames have few pixels to spread many groups'
+// atomics over: a 160 x 120 x 2 x 32 sweep took 42 us with atomics and 36 without.
 constexpr size_t SW_KEY_BYTES = 2 * sizeof(unsigned long long);
+constexpr size_t SW_PART_BYTES = PSW_SWEEP_SCRATCH_BYTES;
+static size_t sweep_ws_bytes(const SweepArgs& a, bool* part) {
+    const size_t npix = (size_t)a.W * a.H, p = 3 * sizeof(float) * (size_t)a.G * npix;
+    *part = p <= SW_PART_BYTES;
+    return *part ? p : npix * SW_KEY_BYTES;
+}
 static int sweep_aggregate_run(SweepArgs& a, int winsize, int fast, void* ws, hipStream_t st) {
     const size_t npix = (size_t)a.W * a.H;
     int rc = PSW_OK;
+    bool part = false;
     if (a.G > 1) {
-        a.top2 = static_cast<unsigned long long*>(ws);
-        rc = psw_fill_u32(reinterpret_cast<uint32_t*>(ws), 0xFFFFFFFFu, 4 * npix, st);
+        (void)sweep_ws_bytes(a, &part);
+        if (part) {
+            a.part = static_cast<float*>(ws);
+        } else {
+            a.top2 = static_cast<unsigned long long*>(ws);
+            rc = psw_fill_u32(reinterpret_cast<uint32_t*>(ws), 0xFFFFFFFFu, 4 * npix, st);
+        }
     }
     if (rc == PSW_OK) rc = launch_sweep(a, winsize, 1, fast != 0, st);
     if (rc == PSW_OK && a.G > 1) {
-        sweep_top2_kernel<<<(unsigned)((npix + 255) / 256), 256, 0, st>>>(a.top2, npix, a.argmin, a.cmin, a.csec);
+        if (part)
+            sweep_merge_kernel<<<(unsigned)((npix + 63) / 64), 256, 0, st>>>(a.part, npix, a.G, a.argmin, a.cmin, a.csec);
+        else
+            sweep_top2_kernel<<<(unsigned)((npix + 255) / 256), 256, 0, st>>>(a.top2, npix, a.argmin, a.cmin, a.csec);
         rc = launch_status("sweep_top2_kernel");
     }
     return rc;
@@ -716,8 +995,33 @@ int psw_sweep_fused_reference(const float* d_ref, const float* d_src, int width,
     a.W = width; a.H = height; a.N = nsrc; a.P = nplanes; a.off = 1;
     a.stdthresh = stdthresh; a.nccthresh = nccthresh; a.zfar = zfar;
     a.depth_out = d_depth_out;
-    sweep_layout(a, false);
-    return launch_sweep(a, winsize, 0, false, S(s));
+    sweep_layout(a, false, sweep_tile_height(), winsize);
+    // One workgroup per (tile, source, plane group), the sources' best keys
+    // from the workspace pool; one per tile, with no workspace, under stream
+    // capture, for one source in few planes, or when the pool has no memory.
+    const size_t npix = (size_t)width * height;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    (void)hipStreamIsCapturing(S(s), &cap);
+    void* ws = nullptr;
+    const int G = (int)std::max(1L, std::min((long)nplanes, SW_TARGET_ITEMS / ((long)a.ntiles * nsrc)));
+    if (cap == hipStreamCaptureStatusNone && nsrc * G > 1 &&
+        workspace_alloc_async(&ws, npix * nsrc * sizeof(unsigned long long), S(s)) != PSW_OK) {
+        (void)hipGetLastError();
+        ws = nullptr;
+    }
+    if (!ws) return launch_sweep(a, winsize, 0, false, S(s));
+    a.top2 = static_cast<unsigned long long*>(ws);
+    a.S = nsrc;
+    a.G = std::min(G, 64);
+    st = psw_fill_u32(static_cast<uint32_t*>(ws), 0u, 2 * npix * nsrc, s);
+    if (st == PSW_OK) st = launch_sweep(a, winsize, 0, false, S(s));
+    if (st == PSW_OK) {
+        sweep_best_depth_kernel<<<(unsigned)((npix + 255) / 256), 256, 0, S(s)>>>(a.top2, npix, nsrc, d_depths, nccthresh,
+                                                                                   zfar, d_depth_out);
+        st = launch_status("sweep_best_depth_kernel");
+    }
+    (void)workspace_free_async(ws, S(s));
+    return st;
 }
 
 int psw_sweep_fused_aggregate(const float* d_ref, const float* d_src, int width, int height, int nsrc,
@@ -732,11 +1036,11 @@ int psw_sweep_fused_aggregate(const float* d_ref, const float* d_src, int width,
     a.W = width; a.H = height; a.N = nsrc; a.P = nplanes; a.off = coord_offset;
     a.stdthresh = stdthresh;
     a.argmin = d_argmin; a.cmin = d_cost_min; a.csec = d_cost_second;
-    sweep_layout(a, true, sweep_tile_height());
-    const size_t npix = (size_t)width * height;
+    sweep_layout(a, true, sweep_tile_height(), winsize);
     void* ws = nullptr;
-    if (a.G > 1) {   // the plane groups' keys, from the library's workspace pool
-        st = workspace_alloc_async(&ws, npix * SW_KEY_BYTES, S(s));
+    if (a.G > 1) {   // the plane groups' results, from the library's workspace pool
+        bool part = false;
+        st = workspace_alloc_async(&ws, sweep_ws_bytes(a, &part), S(s));
         if (st != PSW_OK) return st;
     }
     st = sweep_aggregate_run(a, winsize, fast, ws, S(s));
@@ -758,7 +1062,7 @@ int psw_sweep_fused_aggregate_noalloc(const float* d_ref, const float* d_src, in
     a.W = width; a.H = height; a.N = nsrc; a.P = nplanes; a.off = coord_offset;
     a.stdthresh = stdthresh;
     a.argmin = d_argmin; a.cmin = d_cost_min; a.csec = d_cost_second;
-    sweep_layout(a, true, sweep_tile_height());
+    sweep_layout(a, true, sweep_tile_height(), winsize);
     const size_t key_bytes = (size_t)width * height * SW_KEY_BYTES;
     if (groups > 0) {
         a.G = std::min(groups, std::min(a.P, 64));
@@ -784,7 +1088,16 @@ int psw_sweep_fused_aggregate_batch(const psw_sweep_frame* frames, int nframes, 
     std::vector<SweepArgs> args((size_t)nframes);
     std::vector<int> off((size_t)nframes + 1, 0);
     long total_tiles = 0;
-    const int ty = sweep_tile_height();
+    int ty = sweep_tile_height();
+    if (!ty) {   // the launch has one tile shape: the one with fewer tiles in all
+        long n16 = 0, n32 = 0;
+        for (int f = 0; f < nframes; ++f) {
+            if (frames[f].width < 1 || frames[f].height < 1) continue;   // refused below
+            n16 += sweep_tiles(frames[f].width, frames[f].height, 16);
+            n32 += sweep_tiles(frames[f].width, frames[f].height, 32);
+        }
+        ty = n32 < n16 ? 32 : 16;
+    }
     for (int f = 0; f < nframes; ++f) {
         const psw_sweep_frame& fr = frames[f];
         int st = check_sweep_args(fr.d_ref, fr.d_src, fr.width, fr.height, fr.nsrc, fr.d_H, fr.nplanes, winsize);
@@ -800,13 +1113,13 @@ int psw_sweep_fused_aggregate_batch(const psw_sweep_frame* frames, int nframes, 
         a.W = fr.width; a.H = fr.height; a.N = fr.nsrc; a.P = fr.nplanes; a.off = coord_offset;
         a.stdthresh = stdthresh;
         a.argmin = fr.d_argmin; a.cmin = fr.d_cost_min; a.csec = fr.d_cost_second;
-        sweep_layout(a, false, ty);
+        sweep_layout(a, false, ty, winsize);
         total_tiles += a.ntiles;
     }
     // Plane groups: enough items across the whole batch to fill the GPU
-    // (about 3000 workgroups' worth) unless given.
+    // unless given.
     int G = groups > 0 ? groups
-                       : (int)std::max(1L, (SW_TARGET_ITEMS * 16 / ty + total_tiles / 2) / std::max(1L, total_tiles));
+                       : (int)std::max(1L, (SW_TARGET_ITEMS + total_tiles / 2) / std::max(1L, total_tiles));
     size_t ws_bytes = 0;
     for (int f = 0; f < nframes; ++f) {
         SweepArgs& a = args[(size_t)f];
@@ -851,11 +1164,11 @@ int psw_sweep_fused_aggregate_batch(const psw_sweep_frame* frames, int nframes, 
 #define PSW_SB(r)                                                                                             \
     case r:                                                                                                   \
         if (ty == 32) {                                                                                       \
-            if (fast) sweep_batch_kernel<r, 1, true, 32><<<grid, block, 0, st>>>(d_args, d_off, nframes, total, d_counter); \
-            else sweep_batch_kernel<r, 1, false, 32><<<grid, block, 0, st>>>(d_args, d_off, nframes, total, d_counter); \
+            if (fast) sweep_batch_kernel<r, 1, true, 32, 32><<<grid, block, 0, st>>>(d_args, d_off, nframes, total, d_counter); \
+            else sweep_batch_kernel<r, 1, false, 32, 32><<<grid, block, 0, st>>>(d_args, d_off, nframes, total, d_counter); \
         } else {                                                                                              \
-            if (fast) sweep_batch_kernel<r, 1, true, 16><<<grid, block, 0, st>>>(d_args, d_off, nframes, total, d_counter); \
-            else sweep_batch_kernel<r, 1, false, 16><<<grid, block, 0, st>>>(d_args, d_off, nframes, total, d_counter); \
+            if (fast) sweep_batch_kernel<r, 1, true, 64, 16><<<grid, block, 0, st>>>(d_args, d_off, nframes, total, d_counter); \
+            else sweep_batch_kernel<r, 1, false, 64, 16><<<grid, block, 0, st>>>(d_args, d_off, nframes, total, d_counter); \
         }                                                                                                     \
         break;
             PSW_SB(0) PSW_SB(1) PSW_SB(2) PSW_SB(3) PSW_SB(4) PSW_SB(5) PSW_SB(6) PSW_SB(7)

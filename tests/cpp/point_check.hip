@@ -114,7 +114,42 @@ __global__ void check_kernel(uint64_t n, uint64_t seed, unsigned long long* coun
     atomicAdd(&counts[4], proj);
 }
 
+// div_win (the sweep's window means) against '/': every mantissa, both signs,
+// at the ends and the middle of its range, for one window size.
+template <int WIN>
+__device__ unsigned long long win_mismatches(uint32_t m) {
+    unsigned long long bad = 0;
+    for (int e = -60; e <= 59; e += 17) {
+        const float s = __uint_as_float(((uint32_t)(e + 127) << 23) | m);
+        bad += !same(psw::div_win<WIN>(s), s / (float)WIN);
+        bad += !same(psw::div_win<WIN>(-s), -s / (float)WIN);
+    }
+    return bad;
+}
+
+__global__ void win_kernel(unsigned long long* bad) {
+    unsigned long long b = 0;
+    for (uint32_t m = blockIdx.x * blockDim.x + threadIdx.x; m < (1u << 23); m += gridDim.x * blockDim.x)
+        b += win_mismatches<1>(m) + win_mismatches<3>(m) + win_mismatches<5>(m) + win_mismatches<7>(m) +
+             win_mismatches<9>(m) + win_mismatches<11>(m) + win_mismatches<13>(m) + win_mismatches<15>(m);
+    atomicAdd(bad, b);
+}
+
 }  // namespace
+
+// Mismatches of div_win; below 0: a device error.
+extern "C" long long window_check(void) {
+    unsigned long long *d = nullptr, out = 0;
+    if (hipMalloc(&d, sizeof(out)) != hipSuccess) return -1;
+    long long rc = hipMemset(d, 0, sizeof(out)) == hipSuccess ? 0 : -2;
+    if (rc == 0) {
+        win_kernel<<<2048, 256>>>(d);
+        if (hipGetLastError() != hipSuccess || hipMemcpy(&out, d, sizeof(out), hipMemcpyDeviceToHost) != hipSuccess)
+            rc = -3;
+    }
+    (void)hipFree(d);
+    return rc == 0 ? (long long)out : rc;
+}
 
 extern "C" int point_check(uint64_t n, uint64_t seed, unsigned long long* out) {
     unsigned long long* d = nullptr;

@@ -40,3 +40,12 @@ def test_projection_arithmetic_bit_exact(gpu, seed):
     # the fast quotient path ran (|x| >= 2^-100 and s < 2^40: about 1 case in 8),
     # and dual updates with and without a projection were compared
     assert fast > n // 16 and n // 8 < proj < n - n // 8
+
+
+@pytest.mark.gpu
+def test_window_division_bit_exact(gpu):
+    """The reference-order sweep divides its window sums by the window size
+    with one residual correction: every mantissa, every window size."""
+    lib = ctypes.CDLL(LIB)
+    lib.window_check.restype = ctypes.c_longlong
+    assert lib.window_check() == 0
