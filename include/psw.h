@@ -261,9 +261,8 @@ int psw_sweep_fused_reference(const float* d_ref, const float* d_src, int width,
  * fast = 0: reference-order arithmetic (bit-identical to the float oracle);
  * fast = 1: running window sums, reciprocal scaling and FMA.  With more
  * than one plane group (the default below about 3400 tiles of 1024 pixels;
- * PSW_SWEEP_GROUPS sets it) the groups' results, 12 bytes per pixel and
- * group up to 32 MiB in all, else keys of 16 bytes per pixel, go to the
- * library's stream-ordered workspace pool, which keeps freed blocks for
+ * PSW_SWEEP_GROUPS sets it) the groups' keys, 16 bytes per pixel, come from
+ * the library's stream-ordered workspace pool, which keeps freed blocks for
  * later calls until the process ends. */
 int psw_sweep_fused_aggregate(const float* d_ref, const float* d_src, int width, int height, int nsrc,
                               const float* d_H, int nplanes, int winsize, float stdthresh, int coord_offset,
@@ -277,7 +276,7 @@ int psw_sweep_argmin_depth(float* d_depth, const int32_t* d_argmin, const float*
 /* psw_sweep_fused_aggregate without any device allocation.  No counterpart
  * in the reference: for callers that cannot allocate device memory (code
  * under hipGraph capture, tight serving loops).  The plane groups'
- * results (as above: at most 32 MiB, or 16 bytes per pixel) go to a static
+ * per-pixel keys (16 bytes per pixel at any group count) go to a static
  * device array of PSW_SWEEP_SCRATCH_BYTES (32 MiB, held by every GPU the
  * library runs on until the process ends: frames up to 2^21 pixels) instead
  * of a per-call allocation; outputs are bit-identical to

@@ -62,8 +62,6 @@ struct SweepArgs {
     float* csec;
     unsigned long long* top2;  // ... else every group's best two go to these per-pixel keys [2][H*W];
                                // split reference sweep: best keys [N][H*W]
-    float* part;               // aggregate mode, small frames: each group's best cost, plane and second-best
-                               // cost instead, [3][G][H*W]
 };
 
 // The aggregated sweep's plane groups of one tile run in different
@@ -575,13 +573,7 @@ __device__ __forceinline__ void sweep_item(const SweepArgs& a, const int item) {
             if (!pixel(k, i)) continue;
             const float c1 = got(0, k), c2 = got(2, k);
             const int p = __float_as_int(got(1, k));
-            if (a.G > 1 && a.part) {
-                float* const o = a.part + (size_t)g * npix + i;
-                const size_t plane = (size_t)a.G * npix;
-                o[0] = c1;
-                o[plane] = __int_as_float(p);
-                o[2 * plane] = c2;
-            } else if (a.G > 1) {
+            if (a.G > 1) {
                 sweep_top2_insert(a.top2, npix, i, c1, p, c2);
             } else {
                 a.argmin[i] = p;
@@ -659,60 +651,6 @@ __global__ void sweep_top2_kernel(const unsigned long long* __restrict__ top2, s
     arg[i] = k0 == ~0ull ? -1 : (int32_t)(unsigned)k0;
     cmin[i] = k0 == ~0ull ? inf : sweep_key_cost(k0);
     csec[i] = k1 == ~0ull ? inf : sweep_key_cost(k1);
-}
-
-// Folds the best cost a1 at plane ap and second-best a2 of later planes into
-// c1, p1, c2, as the scan over all planes does.
-__device__ __forceinline__ void merge_bests(float a1, int ap, float a2, float& c1, int& p1, float& c2) {
-    if (a1 < c1) {
-        c2 = a2 < c1 ? a2 : c1;
-        c1 = a1;
-        p1 = ap;
-    } else if (a1 < c2) {
-        c2 = a1;
-    }
-}
-
-// The outputs from the plane groups' own bests (-0 folded into +0, as in the
-// keys).  A wave takes 64 pixels, the four waves of a workgroup a quarter of
-// the groups each, eight loads of each array in flight: with one thread to a
-// pixel's groups the loads of a small frame were one long chain.
-__global__ __launch_bounds__(256) void sweep_merge_kernel(const float* __restrict__ part, size_t npix, int G,
-                                                          int32_t* __restrict__ arg, float* __restrict__ cmin,
-                                                          float* __restrict__ csec) {
-    __shared__ float s1[4][64], s2[4][64];
-    __shared__ int sp[4][64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const size_t i = (size_t)blockIdx.x * 64 + lane, plane = (size_t)G * npix;
-    float c1 = __builtin_inff(), c2 = c1;
-    int p1 = -1;
-    if (i < npix) {
-        const int g1 = (w + 1) * G / 4;
-        for (int g = w * G / 4; g < g1; g += 8) {
-            float a1[8], a2[8];
-            int ap[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const float* const o = part + (size_t)min(g + k, g1 - 1) * npix + i;
-                a1[k] = o[0];
-                ap[k] = __float_as_int(o[plane]);
-                a2[k] = o[2 * plane];
-            }
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-                if (g + k < g1) merge_bests(a1[k], ap[k], a2[k], c1, p1, c2);
-        }
-    }
-    s1[w][lane] = c1;
-    sp[w][lane] = p1;
-    s2[w][lane] = c2;
-    __syncthreads();
-    if (w != 0 || i >= npix) return;
-#pragma unroll
-    for (int k = 1; k < 4; ++k) merge_bests(s1[k][lane], sp[k][lane], s2[k][lane], c1, p1, c2);
-    arg[i] = p1;
-    cmin[i] = c1 + 0.0f;
-    csec[i] = c2 + 0.0f;
 }
 
 // ---- FP64 homographies -----------------------------------------------------
@@ -838,7 +776,7 @@ static int launch_sweep(SweepArgs a, int winsize, int mode, bool fast, hipStream
 // Measured over 30 sizes from 112 x 88 to 981 x 553 (1.36 times as fast on
 // average as 32 x 16 tiles with 14400 workgroups): 6, 9 and 12 steps are
 // within 3 % of each other on average, and with 9 / 6 no size is slower by
-// more than 3 %.
+// more than 10 % (114 x 87, where the whole call takes 45 us).
 // PSW_SWEEP_GROUPS overrides the choice (up to 64).
 constexpr long SW_TARGET_ITEMS = 5120, SW_SLOTS = 1280;
 // The tile shape: PSW_SWEEP_TY 16 (64 x 16) or 32 (32 x 32), else 0 for the
@@ -865,7 +803,7 @@ static void sweep_layout(SweepArgs& a, bool allow_groups, int ty, int winsize) {
     long G = std::min((SW_TARGET_ITEMS + nt / 2) / nt, std::max((long)a.N * a.P / (winsize > 9 ? 6 : 9), 256 / nt));
     if (nt * G > SW_SLOTS && nt * G < 3 * SW_SLOTS) G = nt * G / SW_SLOTS * SW_SLOTS / nt;
     if (const char* e = getenv("PSW_SWEEP_GROUPS")) G = std::min(atoi(e), 64);
-    a.G = (int)std::max(1L, std::min(G, (long)std::min(a.P, 128)));
+    a.G = (int)std::max(1L, std::min(G, (long)std::min(a.P, 64)));
 }
 
 static int check_sweep_args(const float* d_ref, const float* d_src, int width, int height, int nsrc,
@@ -914,38 +852,22 @@ static int scratch_address(void** out) {
     return PSW_OK;
 }
 
-// The aggregated sweep's launch and, with plane groups, their workspace `ws`
-// of sweep_ws_bytes: the groups' own bests, merged after, where those fit
-// SW_PART_BYTES (frames up to 320 x 240 at the default group count); else the
-// per-pixel keys (SW_KEY_BYTES per pixel: cleared first, turned into the
-// outputs after).  Small frames have few pixels to spread many groups'
-// atomics over: a 160 x 120 x 2 x 32 sweep took 42 us with atomics and 36 without.
+// The aggregated sweep's launch and, with plane groups, the per-pixel keys
+// in `ws` (SW_KEY_BYTES per pixel: cleared first, turned into the outputs
+// after).  (The groups' bests as partial results, merged by one launch, took
+// 1 to 3 us less on small frames, but workspaces above 2 MB cost the first
+// call on them 30 us.)
 constexpr size_t SW_KEY_BYTES = 2 * sizeof(unsigned long long);
-constexpr size_t SW_PART_BYTES = PSW_SWEEP_SCRATCH_BYTES;
-static size_t sweep_ws_bytes(const SweepArgs& a, bool* part) {
-    const size_t npix = (size_t)a.W * a.H, p = 3 * sizeof(float) * (size_t)a.G * npix;
-    *part = p <= SW_PART_BYTES;
-    return *part ? p : npix * SW_KEY_BYTES;
-}
 static int sweep_aggregate_run(SweepArgs& a, int winsize, int fast, void* ws, hipStream_t st) {
     const size_t npix = (size_t)a.W * a.H;
     int rc = PSW_OK;
-    bool part = false;
     if (a.G > 1) {
-        (void)sweep_ws_bytes(a, &part);
-        if (part) {
-            a.part = static_cast<float*>(ws);
-        } else {
-            a.top2 = static_cast<unsigned long long*>(ws);
-            rc = psw_fill_u32(reinterpret_cast<uint32_t*>(ws), 0xFFFFFFFFu, 4 * npix, st);
-        }
+        a.top2 = static_cast<unsigned long long*>(ws);
+        rc = psw_fill_u32(reinterpret_cast<uint32_t*>(ws), 0xFFFFFFFFu, 4 * npix, st);
     }
     if (rc == PSW_OK) rc = launch_sweep(a, winsize, 1, fast != 0, st);
     if (rc == PSW_OK && a.G > 1) {
-        if (part)
-            sweep_merge_kernel<<<(unsigned)((npix + 63) / 64), 256, 0, st>>>(a.part, npix, a.G, a.argmin, a.cmin, a.csec);
-        else
-            sweep_top2_kernel<<<(unsigned)((npix + 255) / 256), 256, 0, st>>>(a.top2, npix, a.argmin, a.cmin, a.csec);
+        sweep_top2_kernel<<<(unsigned)((npix + 255) / 256), 256, 0, st>>>(a.top2, npix, a.argmin, a.cmin, a.csec);
         rc = launch_status("sweep_top2_kernel");
     }
     return rc;
@@ -1037,10 +959,10 @@ int psw_sweep_fused_aggregate(const float* d_ref, const float* d_src, int width,
     a.stdthresh = stdthresh;
     a.argmin = d_argmin; a.cmin = d_cost_min; a.csec = d_cost_second;
     sweep_layout(a, true, sweep_tile_height(), winsize);
+    const size_t npix = (size_t)width * height;
     void* ws = nullptr;
-    if (a.G > 1) {   // the plane groups' results, from the library's workspace pool
-        bool part = false;
-        st = workspace_alloc_async(&ws, sweep_ws_bytes(a, &part), S(s));
+    if (a.G > 1) {   // the plane groups' keys, from the library's workspace pool
+        st = workspace_alloc_async(&ws, npix * SW_KEY_BYTES, S(s));
         if (st != PSW_OK) return st;
     }
     st = sweep_aggregate_run(a, winsize, fast, ws, S(s));

@@ -1,6 +1,6 @@
 """The sweep's split of the work at the sizes where it can go wrong: frames
 that cut the 64 x 16 and 32 x 32 tiles, windows of every size, one source,
-plane groups merged from partial results and through per-pixel keys, steps
+plane groups merged through per-pixel keys, steps
 whose tile lies inside the source and steps whose tile does not, textureless
 and zero regions (the reference order's general divisions), values near the
 ends of the exponent range, and non-finite pixels.
