@@ -43,6 +43,17 @@ __host__ __device__ inline uint16_t f2bf(float f) {
 }
 __host__ __device__ inline float bf2f(uint16_t h) { return __builtin_bit_cast(float, (uint32_t)h << 16); }
 
+// v's bf16 values where those of y are positive, else 0.
+__device__ inline uint32_t mask_bf16x2(uint32_t v, uint32_t y) {
+    const uint32_t lo = bf2f((uint16_t)y) > 0.f ? 0xffffu : 0u;
+    const uint32_t hi = bf2f((uint16_t)(y >> 16)) > 0.f ? 0xffff0000u : 0u;
+    return v & (lo | hi);
+}
+__device__ inline uint4 mask_bf16x8(uint4 v, uint4 y) {
+    return make_uint4(mask_bf16x2(v.x, y.x), mask_bf16x2(v.y, y.y), mask_bf16x2(v.z, y.z), mask_bf16x2(v.w, y.w));
+}
+__device__ inline uint32_t pack_bf16x2(float a, float b) { return f2bf(a) | ((uint32_t)f2bf(b) << 16); }
+
 constexpr int UN_LAYERS = 14;
 constexpr int UN_IN = 8;     // input channels (5 used)
 constexpr int UN_OUT = 8;    // output channels
@@ -64,9 +75,17 @@ struct ConvK {
     const uint16_t* xb;   // [B][H/2][W/2][cb] (nearest-upsampled), or null
     const uint16_t* wp;   // packed weights [conv_chunks(ca + cb)][NB][64][8]
     const float* bias;    // [cout] or null
-    void* y;              // [B][H][W][cout]: bf16 (relu) or fp32
+    const uint16_t* mask; // [B][H][W][cout] activations (CONV_MASKED)
+    void* y;              // [B][H][W][cout]: bf16 or fp32, see ConvOut
     int ca, cb, cout, B, H, W, kchunks;
 };
+
+// What a convolution writes: FP32, bf16 ReLU, or bf16 of the FP32 value where
+// the activation `mask` is positive and 0 elsewhere.  The last is a data
+// gradient that goes straight on to the layer below as its dZ: FP32
+// gradients and a pass over them to mask and round (19 us on average, ten
+// times per training step of 8 x 256 x 256) never reach memory.
+enum ConvOut { CONV_F32, CONV_RELU, CONV_MASKED };
 
 // Output tile of one block: 8 rows x 32 columns, four waves of 2 rows each
 // (4 MFMA row blocks of 16 pixels per wave).  The input tile with its
@@ -148,7 +167,7 @@ __device__ __forceinline__ void conv_slab(f32x4 (&acc)[4][NBL], const uint16_t* 
 // over several blocks so that a launch still has enough of them.  The
 // results go through LDS, 16 channels at a time, so that every thread
 // stores whole 16-byte runs of one pixel's channels.
-template <int NBL, bool RELU_BF16>
+template <int NBL, int OUT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NBL == 1 ? 4 : 1)))
 void conv3x3_kernel(ConvK a) {
     constexpr int NPIX = CT_HH * CT_HW;               // staged pixels (tile + halo)
@@ -261,21 +280,27 @@ void conv3x3_kernel(ConvK a) {
         const int ch0 = (nb0 + nb) * 16;
         const float bias = a.bias ? a.bias[ch0 + col] : 0.f;
         __syncthreads();                                   // sx is free (K loop or previous block of channels)
-        if (RELU_BF16) {
+        if (OUT != CONV_F32) {
             uint16_t* so = sx;
 #pragma unroll
             for (int m = 0; m < 4; ++m)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int q = (wave * 2 + (m >> 1)) * CT_TW + (m & 1) * 16 + 4 * jg + i;
-                    so[q * 24 + col] = f2bf(fmaxf(acc[m][nb][i] + bias, 0.f));
+                    so[q * 24 + col] = f2bf(OUT == CONV_RELU ? fmaxf(acc[m][nb][i] + bias, 0.f) : acc[m][nb][i]);
                 }
             __syncthreads();
             if (out) {
                 const uint4* src = reinterpret_cast<const uint4*>(&so[t * 24]);
                 uint4* dst = reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(a.y) + p * a.cout + ch0);
-                dst[0] = src[0];
-                dst[1] = src[1];
+                uint4 v0 = src[0], v1 = src[1];
+                if (OUT == CONV_MASKED) {
+                    const uint4* mk = reinterpret_cast<const uint4*>(a.mask + p * a.cout + ch0);
+                    v0 = mask_bf16x8(v0, mk[0]);
+                    v1 = mask_bf16x8(v1, mk[1]);
+                }
+                dst[0] = v0;
+                dst[1] = v1;
             }
         } else {
             float* so = reinterpret_cast<float*>(sx);
@@ -303,33 +328,44 @@ void conv3x3_kernel(ConvK a) {
 // cout channels of dZ, N = cin, with W'[tap'][co][ci] = W[8 - tap'][ci][co]
 // (the data gradient is the forward convolution of dZ with the
 // 180-degree-rotated, transposed kernel).
-__global__ void pack_w_kernel(const float* __restrict__ w, int cin, int cout, int flip, int kchunks, int NB,
-                              uint16_t* __restrict__ wp) {
-    const long n_el = (long)kchunks * NB * 512;
-    const int C = flip ? cout : cin, NO = flip ? cin : cout;
-    for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < n_el; idx += (long)gridDim.x * blockDim.x) {
-        const int j = (int)(idx & 7), l = (int)((idx >> 3) & 63);
-        const long r = idx >> 9;
-        const int nb = (int)(r % NB), kc = (int)(r / NB);
-        const int slab = kc / 9, local = kc - slab * 9;
-        const int c0 = 32 * slab;
-        const int g8 = (C - c0 < 32 ? C - c0 : 32) >> 3;
-        const int gi = 4 * local + (l >> 4), n = nb * 16 + (l & 15);
-        float v = 0.f;
-        if (c0 < C && gi < 9 * g8 && n < NO) {
-            const int tap = gi / g8, c = c0 + (gi - tap * g8) * 8 + j;
-            if (!flip) v = w[((long)tap * cin + c) * cout + n];
-            else v = w[((long)(8 - tap) * cin + n) * cout + c];
-        }
-        wp[idx] = f2bf(v);
+struct PackK {
+    const float* w;
+    uint16_t* wp;
+    int cin, cout, flip, kchunks, NB;
+};
+__device__ __forceinline__ void pack_w(const PackK& a, long idx) {
+    const int C = a.flip ? a.cout : a.cin, NO = a.flip ? a.cin : a.cout;
+    const int j = (int)(idx & 7), l = (int)((idx >> 3) & 63);
+    const int r = (int)(idx >> 9);
+    const int nb = r % a.NB, kc = r / a.NB;
+    const int slab = kc / 9, local = kc - slab * 9;
+    const int c0 = 32 * slab;
+    const int g8 = (C - c0 < 32 ? C - c0 : 32) >> 3;
+    const int gi = 4 * local + (l >> 4), n = nb * 16 + (l & 15);
+    float v = 0.f;
+    if (c0 < C && gi < 9 * g8 && n < NO) {
+        const int tap = gi / g8, c = c0 + (gi - tap * g8) * 8 + j;
+        if (!a.flip) v = a.w[((long)tap * a.cin + c) * a.cout + n];
+        else v = a.w[((long)(8 - tap) * a.cin + n) * a.cout + c];
     }
+    a.wp[idx] = f2bf(v);
+}
+__global__ void pack_w_kernel(PackK a) {
+    const long n_el = (long)a.kchunks * a.NB * 512;
+    for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < n_el; idx += (long)gridDim.x * blockDim.x)
+        pack_w(a, idx);
 }
 
-// dZ = bf16(g * (y > 0)) for a ReLU output y.
-__global__ void relu_bwd_kernel(const uint16_t* __restrict__ y, const float* __restrict__ g, uint16_t* __restrict__ dz,
-                                long n) {
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
-        dz[i] = f2bf(bf2f(y[i]) > 0.f ? g[i] : 0.f);
+// Every layer's packs in one launch (blockIdx.y: the pack), instead of 27
+// launches of 3.6 us after each Adam step.
+struct PackAllK {
+    PackK p[2 * UN_LAYERS];
+};
+__global__ void pack_all_kernel(PackAllK a) {
+    const PackK& k = a.p[blockIdx.y];
+    const long n_el = (long)k.kchunks * k.NB * 512;
+    for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < n_el; idx += (long)gridDim.x * blockDim.x)
+        pack_w(k, idx);
 }
 
 struct WgK {
@@ -341,14 +377,38 @@ struct WgK {
 };
 
 // Weight (and bias) gradient: dW[k][n] = sum_p Xcol[p][k] dZ[p][n], with
-// k = 9 C the bias row (Xcol = 1).  Block: 64 k-rows x cout over one chunk
-// of pixels, 32 pixels per step, both operands transposed through LDS so
-// that each MFMA lane reads 8 consecutive pixels.  Chunk partials are summed
-// in a fixed order by wgrad_reduce_kernel (deterministic).
+// k = 9 C the bias row (Xcol = 1).  Block: 128 k-rows x cout over one chunk
+// of pixels, 128 pixels per step, both operands transposed through LDS so
+// that each MFMA lane reads 8 consecutive pixels (row stride 272 bytes: the
+// 16 rows of one read hit disjoint banks).  A thread loads 8 channels of 4
+// neighbouring pixels and writes 8-byte runs of 4 pixels of one channel; the
+// next step's loads are issued before the current products.  Each wave has
+// two 16-row blocks, so that a B fragment read from LDS feeds two products.
+// Chunk partials are summed in a fixed order by wgrad_reduce_kernel
+// (deterministic).
+// Bound by the transposition's LDS traffic and by latency, not by the matrix
+// cores: WGRAD_FIGURES
+constexpr int WG_PX = 128, WG_ST = WG_PX + 8, WG_MR = 2, WG_K = 64 * WG_MR;
+
+// 4 pixels x 8 channels -> per channel, its 4 pixels.
+__device__ __forceinline__ void store_transposed(const uint4 (&v)[4], uint16_t* s, int row0, int px) {
+    const uint32_t* d[4] = {&v[0].x, &v[1].x, &v[2].x, &v[3].x};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const uint2 even = make_uint2((d[0][c] & 0xffffu) | (d[1][c] << 16), (d[2][c] & 0xffffu) | (d[3][c] << 16));
+        const uint2 odd =
+            make_uint2((d[0][c] >> 16) | (d[1][c] & 0xffff0000u), (d[2][c] >> 16) | (d[3][c] & 0xffff0000u));
+        *reinterpret_cast<uint2*>(&s[(row0 + 2 * c) * WG_ST + px]) = even;
+        *reinterpret_cast<uint2*>(&s[(row0 + 2 * c + 1) * WG_ST + px]) = odd;
+    }
+}
+
 template <int NB>
 __global__ __launch_bounds__(256) void wgrad_kernel(WgK a) {
-    __shared__ __align__(16) uint16_t sA[64][40];
-    __shared__ __align__(16) uint16_t sB[NB * 16][40];
+    constexpr int NA = WG_K / 8 * (WG_PX / 4) / 256;          // A pieces (8 channels x 4 pixels) per thread
+    constexpr int NBP = (NB * 2 * (WG_PX / 4) + 255) / 256;   // B pieces per thread
+    __shared__ __align__(16) uint16_t sA[WG_K * WG_ST];
+    __shared__ __align__(16) uint16_t sB[NB * 16 * WG_ST];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int C = a.ca + a.cb, Kw = 9 * C;
     const long NP = (long)a.B * a.H * a.W;
@@ -356,103 +416,193 @@ __global__ __launch_bounds__(256) void wgrad_kernel(WgK a) {
     const long p_begin = (long)chunk * a.chunk_px;
     const long p_end = p_begin + a.chunk_px < NP ? p_begin + a.chunk_px : NP;
     const int Hh = a.H >> 1, Wh = a.W >> 1;
-    f32x4 acc[NB];
+    const int px = (t & 31) * 4;
+    f32x4 acc[WG_MR][NB];
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (long p0 = p_begin; p0 < p_end; p0 += 32) {
-        {
-            const long p = p0 + (t & 31);
-            const int k0 = ktile * 64 + (t >> 5) * 8;
-            uint4 v = make_uint4(0u, 0u, 0u, 0u);
-            if (p < p_end) {
-                if (k0 < Kw) {
-                    const int tap = k0 / C, c0 = k0 - (k0 / C) * C;
-                    const int x = (int)(p % a.W);
-                    const long tt = p / a.W;
-                    const int y = (int)(tt % a.H), b = (int)(tt / a.H);
-                    const int yy = y + tap / 3 - 1, xx = x + tap % 3 - 1;
-                    if (yy >= 0 && yy < a.H && xx >= 0 && xx < a.W) {
-                        if (c0 < a.ca)
-                            v = *reinterpret_cast<const uint4*>(a.xa + (((long)b * a.H + yy) * a.W + xx) * a.ca + c0);
+    for (int m = 0; m < WG_MR; ++m)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) acc[m][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // this thread's A pieces: tap offset and channel group, fixed over the chunk
+    int dy[NA], dx[NA], c0[NA];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+        const int k0 = ktile * WG_K + ((t >> 5) + 8 * i) * 8;
+        const int tap = k0 / C;
+        c0[i] = k0 < Kw ? k0 - tap * C : k0 == Kw ? -1 : -2;   // -1: the bias row, -2: past the end
+        dy[i] = tap / 3 - 1;
+        dx[i] = tap % 3 - 1;
+    }
+    // position of this thread's first pixel, advanced by WG_PX per step
+    int px0, py0, pb0;
+    {
+        const long r = (p_begin + px) / a.W;
+        px0 = (int)(p_begin + px - r * a.W);
+        pb0 = (int)(r / a.H);
+        py0 = (int)(r - (long)pb0 * a.H);
+    }
+    const int sx = WG_PX % a.W, sy = WG_PX / a.W;
+    uint4 va[NA][4], vb[NBP][4];
+    auto load = [&](long p0) {
+        int x[4], y[4], b[4];
+        const long p = p0 + px;
+        x[0] = px0; y[0] = py0; b[0] = pb0;
+        px0 += sx;
+        py0 += sy + (px0 >= a.W ? 1 : 0);
+        px0 -= px0 >= a.W ? a.W : 0;
+        while (py0 >= a.H) { py0 -= a.H; ++pb0; }
+#pragma unroll
+        for (int j = 1; j < 4; ++j) {
+            const bool wx = x[j - 1] + 1 == a.W, wy = wx && y[j - 1] + 1 == a.H;
+            x[j] = wx ? 0 : x[j - 1] + 1;
+            y[j] = wy ? 0 : y[j - 1] + (wx ? 1 : 0);
+            b[j] = b[j - 1] + (wy ? 1 : 0);
+        }
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                uint4 v = make_uint4(0u, 0u, 0u, 0u);
+                if (p + j < p_end && c0[i] >= -1) {
+                    const int yy = y[j] + dy[i], xx = x[j] + dx[i];
+                    if (c0[i] < 0) {
+                        v.x = 0x3f80u;  // bias row: 1.0 in bf16
+                    } else if (yy >= 0 && yy < a.H && xx >= 0 && xx < a.W) {
+                        if (c0[i] < a.ca)
+                            v = *reinterpret_cast<const uint4*>(a.xa + (((long)b[j] * a.H + yy) * a.W + xx) * a.ca +
+                                                                c0[i]);
                         else
                             v = *reinterpret_cast<const uint4*>(
-                                a.xb + (((long)b * Hh + (yy >> 1)) * Wh + (xx >> 1)) * a.cb + (c0 - a.ca));
+                                a.xb + (((long)b[j] * Hh + (yy >> 1)) * Wh + (xx >> 1)) * a.cb + (c0[i] - a.ca));
                     }
-                } else if (k0 == Kw) {
-                    v.x = 0x3f80u;  // bias row: 1.0 in bf16
                 }
+                va[i][j] = v;
             }
-            const uint16_t* e = reinterpret_cast<const uint16_t*>(&v);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) sA[(t >> 5) * 8 + j][t & 31] = e[j];
-        }
-        for (int q = t; q < NB * 2 * 32; q += 256) {
-            const int pxl = q & 31, cg = q >> 5;
-            const long p = p0 + pxl;
-            uint4 v = make_uint4(0u, 0u, 0u, 0u);
-            if (p < p_end) v = *reinterpret_cast<const uint4*>(a.dz + p * a.cout + cg * 8);
-            const uint16_t* e = reinterpret_cast<const uint16_t*>(&v);
+        for (int i = 0; i < NBP; ++i) {
+            const int cg = (t >> 5) + 8 * i;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) sB[cg * 8 + j][pxl] = e[j];
+            for (int j = 0; j < 4; ++j)
+                vb[i][j] = cg < NB * 2 && p + j < p_end
+                               ? *reinterpret_cast<const uint4*>(a.dz + (p + j) * a.cout + cg * 8)
+                               : make_uint4(0u, 0u, 0u, 0u);
         }
+    };
+    load(p_begin);
+    for (long p0 = p_begin; p0 < p_end; p0 += WG_PX) {
+        if (p0 > p_begin) __syncthreads();   // the previous step's reads are done
+#pragma unroll
+        for (int i = 0; i < NA; ++i) store_transposed(va[i], sA, ((t >> 5) + 8 * i) * 8, px);
+#pragma unroll
+        for (int i = 0; i < NBP; ++i)
+            if ((t >> 5) + 8 * i < NB * 2) store_transposed(vb[i], sB, ((t >> 5) + 8 * i) * 8, px);
         __syncthreads();
-        const bf16x8 av = *reinterpret_cast<const bf16x8*>(&sA[wave * 16 + (lane & 15)][(lane >> 4) * 8]);
+        if (p0 + WG_PX < p_end) load(p0 + WG_PX);
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-            const bf16x8 bv = *reinterpret_cast<const bf16x8*>(&sB[nb * 16 + (lane & 15)][(lane >> 4) * 8]);
-            acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc[nb], 0, 0, 0);
+        for (int ks = 0; ks < WG_PX / 32; ++ks) {
+            const int o = ks * 32 + (lane >> 4) * 8;
+            bf16x8 av[WG_MR];
+#pragma unroll
+            for (int m = 0; m < WG_MR; ++m)
+                av[m] = *reinterpret_cast<const bf16x8*>(&sA[((wave * WG_MR + m) * 16 + (lane & 15)) * WG_ST + o]);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                const bf16x8 bv = *reinterpret_cast<const bf16x8*>(&sB[(nb * 16 + (lane & 15)) * WG_ST + o]);
+#pragma unroll
+                for (int m = 0; m < WG_MR; ++m)
+                    acc[m][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[m], bv, acc[m][nb], 0, 0, 0);
+            }
         }
-        __syncthreads();
     }
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
+    for (int m = 0; m < WG_MR; ++m)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int k = ktile * 64 + wave * 16 + 4 * (lane >> 4) + i;
-            if (k < a.Kext) a.part[((long)chunk * a.Kext + k) * a.cout + nb * 16 + (lane & 15)] = acc[nb][i];
-        }
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int k = ktile * WG_K + (wave * WG_MR + m) * 16 + 4 * (lane >> 4) + i;
+                if (k < a.Kext)
+                    a.part[((long)chunk * a.Kext + k) * a.cout + nb * 16 + (lane & 15)] = acc[m][nb][i];
+            }
 }
 
-__global__ void wgrad_reduce_kernel(const float* __restrict__ part, int nchunks, long n, float* __restrict__ out) {
+// Sums the chunks' partials in a fixed order: four waves take a quarter of
+// the chunks each for 64 entries, eight loads in flight, then add up.  (One
+// thread per entry walking all chunks had too few threads to hide its
+// loads: 42 us a call on average, now REDUCE_FIGURES.)
+__global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float* __restrict__ part, int nchunks, long n,
+                                                           float* __restrict__ out) {
+    __shared__ float ss[4][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const long i = (long)blockIdx.x * 64 + lane;
+    float s = 0.f;
+    if (i < n) {
+        const int c1 = (w + 1) * nchunks / 4;
+        for (int c = w * nchunks / 4; c < c1; c += 8) {
+            float v[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[k] = c + k < c1 ? part[(long)(c + k) * n + i] : 0.f;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) s += v[k];
+        }
+    }
+    ss[w][lane] = s;
+    __syncthreads();
+    if (w == 0 && i < n) out[i] = (ss[0][lane] + ss[1][lane]) + (ss[2][lane] + ss[3][lane]);
+}
+
+// The two other ways a gradient reaches a layer's dZ = bf16(g (y > 0)), each
+// one pass, 8 channels per thread, from the FP32 data gradient `tmp`
+// [B][H][W][ca + cb] of a concatenated input [A | up B]:
+// dZ of B (coarse): g = sum over the 2x2 children of tmp[:, ca:].
+__global__ void up_bwd_kernel(const float* __restrict__ tmp, int ca, int cb, int B, int H, int W,
+                              const uint16_t* __restrict__ y, uint16_t* __restrict__ dz) {
+    const int C = ca + cb, G = cb >> 3, Hh = H >> 1, Wh = W >> 1;
+    const long n = (long)B * Hh * Wh * G;
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        float s = 0.f;
-        for (int c = 0; c < nchunks; ++c) s += part[(long)c * n + i];
-        out[i] = s;
-    }
-}
-
-// Data gradient of a concatenated input [A | up B]: g_a = tmp[:, :ca];
-// g_b (coarse) = sum over the 2x2 children of tmp[:, ca:].
-__global__ void concat_bwd_kernel(const float* __restrict__ tmp, int ca, int cb, int B, int H, int W,
-                                  float* __restrict__ ga, float* __restrict__ gb) {
-    const int C = ca + cb;
-    const long na = (long)B * H * W * ca;
-    const int Hh = H >> 1, Wh = W >> 1;
-    const long nb = (long)B * Hh * Wh * cb;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < na + nb; i += (long)gridDim.x * blockDim.x) {
-        if (i < na) {
-            const long p = i / ca;
-            const int c = (int)(i - p * ca);
-            ga[i] = tmp[p * C + c];
-        } else {
-            const long j = i - na;
-            const long q = j / cb;
-            const int c = (int)(j - q * cb);
-            const int x = (int)(q % Wh);
-            const long tt = q / Wh;
-            const int y = (int)(tt % Hh), b = (int)(tt / Hh);
-            float s = 0.f;
-            for (int dy = 0; dy < 2; ++dy)
-                for (int dx = 0; dx < 2; ++dx) {
-                    const long p = ((long)b * H + 2 * y + dy) * W + 2 * x + dx;
-                    s += tmp[p * C + ca + c];
-                }
-            gb[j] = s;
+        const long q = i / G;
+        const int c = (int)(i - q * G) * 8;
+        const int x = (int)(q % Wh);
+        const long tt = q / Wh;
+        const int yy = (int)(tt % Hh), b = (int)(tt / Hh);
+        float s[8] = {};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float4* t4 = reinterpret_cast<const float4*>(
+                tmp + (((long)b * H + 2 * yy + (k >> 1)) * W + 2 * x + (k & 1)) * C + ca + c);
+            const float4 u = t4[0], v = t4[1];
+            s[0] += u.x; s[1] += u.y; s[2] += u.z; s[3] += u.w;
+            s[4] += v.x; s[5] += v.y; s[6] += v.z; s[7] += v.w;
         }
+        const uint4 d = make_uint4(pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3]), pack_bf16x2(s[4], s[5]),
+                                   pack_bf16x2(s[6], s[7]));
+        reinterpret_cast<uint4*>(dz)[i] = mask_bf16x8(d, reinterpret_cast<const uint4*>(y)[i]);
+    }
+}
+// dZ of A, which is also average-pooled into the next level:
+// g = tmp[:, :ca] + gpool / 4.
+__global__ void skip_bwd_kernel(const float* __restrict__ tmp, int ca, int cb, int B, int H, int W,
+                                const float* __restrict__ gpool, const uint16_t* __restrict__ y,
+                                uint16_t* __restrict__ dz) {
+    const int C = ca + cb, G = ca >> 3, Hh = H >> 1, Wh = W >> 1;
+    const long n = (long)B * H * W * G;
+    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+        const long p = i / G;
+        const int c = (int)(i - p * G) * 8;
+        const int x = (int)(p % W);
+        const long tt = p / W;
+        const int yy = (int)(tt % H), b = (int)(tt / H);
+        const float* g = tmp + p * C + c;
+        const float* q = gpool + (((long)b * Hh + (yy >> 1)) * Wh + (x >> 1)) * ca + c;
+        float s[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) s[k] = g[k] + 0.25f * q[k];
+        const uint4 d = make_uint4(pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3]), pack_bf16x2(s[4], s[5]),
+                                   pack_bf16x2(s[6], s[7]));
+        reinterpret_cast<uint4*>(dz)[i] = mask_bf16x8(d, reinterpret_cast<const uint4*>(y)[i]);
     }
 }
 
-// 2x2 average pooling (bf16 -> bf16, FP32 sum) and its backward (accumulate).
+// 2x2 average pooling (bf16 -> bf16, FP32 sum).
 __global__ void pool_fwd_kernel(const uint16_t* __restrict__ x, int C, int B, int H, int W, uint16_t* __restrict__ y) {
     const int Hh = H >> 1, Wh = W >> 1;
     const long n = (long)B * Hh * Wh * C;
@@ -465,19 +615,6 @@ __global__ void pool_fwd_kernel(const uint16_t* __restrict__ x, int C, int B, in
         const long p = ((long)b * H + 2 * yy) * W + 2 * xx;
         const float s = (bf2f(x[p * C + c]) + bf2f(x[(p + 1) * C + c])) + (bf2f(x[(p + W) * C + c]) + bf2f(x[(p + W + 1) * C + c]));
         y[i] = f2bf(0.25f * s);
-    }
-}
-
-__global__ void pool_bwd_kernel(const float* __restrict__ gy, int C, int B, int H, int W, float* __restrict__ gx) {
-    const long n = (long)B * H * W * C;
-    const int Hh = H >> 1, Wh = W >> 1;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        const long p = i / C;
-        const int c = (int)(i - p * C);
-        const int x = (int)(p % W);
-        const long tt = p / W;
-        const int y = (int)(tt % H), b = (int)(tt / H);
-        gx[i] += 0.25f * gy[(((long)b * Hh + (y >> 1)) * Wh + (x >> 1)) * C + c];
     }
 }
 
@@ -508,11 +645,12 @@ __global__ void head_fwd_kernel(const uint16_t* __restrict__ x, const float* __r
     for (int k = 0; k < UN_OUT; ++k) out[p * UN_OUT + k] = o[k];
 }
 
-// Head backward: g_x[p][c] = sum_o g[p][o] W[c][o]; per-chunk partials of
+// Head backward: dZ of the last layer from g_x[p][c] = sum_o g[p][o] W[c][o]
+// (masked by x > 0, bf16); per-chunk partials of
 // dW[c][o] = sum_p x[p][c] g[p][o] and db[o] = sum_p g[p][o].
 __global__ __launch_bounds__(256) void head_bwd_kernel(const uint16_t* __restrict__ x, const float* __restrict__ g,
                                                        const float* __restrict__ w, long NP, int chunk_px,
-                                                       float* __restrict__ gx, float* __restrict__ part) {
+                                                       uint16_t* __restrict__ dz, float* __restrict__ part) {
     __shared__ float sw[UN_HEAD_IN * UN_OUT];
     __shared__ float sx[64][UN_HEAD_IN + 1];
     __shared__ float sg[64][UN_OUT + 1];
@@ -545,7 +683,7 @@ __global__ __launch_bounds__(256) void head_bwd_kernel(const uint16_t* __restric
                 float s = 0.f;
 #pragma unroll
                 for (int k = 0; k < UN_OUT; ++k) s += sg[r][k] * sw[cc * UN_OUT + k];
-                gx[p * UN_HEAD_IN + cc] = s;
+                dz[p * UN_HEAD_IN + cc] = sx[r][cc] > 0.f ? f2bf(s) : (uint16_t)0;
             }
         }
         __syncthreads();
@@ -678,7 +816,7 @@ static inline unsigned grid_for(long n, int per = 256) {
 
 // Output-channel split: levels with few tiles give each block fewer
 // 16-channel output blocks (NBL), so that a launch has about 1000 blocks.
-template <bool RELU>
+template <int OUT>
 static void launch_conv(const ConvK& a, int NB, hipStream_t st) {
     const long tiles = (long)a.B * ((a.H + CT_TH - 1) / CT_TH) * ((a.W + CT_TW - 1) / CT_TW);
     int nbl = NB;
@@ -687,7 +825,7 @@ static void launch_conv(const ConvK& a, int NB, hipStream_t st) {
     const dim3 grd((unsigned)tiles, (unsigned)(NB / nbl));
     switch (nbl) {
 #define PSW_CONV_CASE(n) \
-    case n: conv3x3_kernel<n, RELU><<<grd, 256, 0, st>>>(a); break;
+    case n: conv3x3_kernel<n, OUT><<<grd, 256, 0, st>>>(a); break;
         PSW_CONV_CASE(1) PSW_CONV_CASE(2) PSW_CONV_CASE(3) PSW_CONV_CASE(4) PSW_CONV_CASE(5) PSW_CONV_CASE(6)
         PSW_CONV_CASE(7) PSW_CONV_CASE(10)
 #undef PSW_CONV_CASE
@@ -710,7 +848,7 @@ static int chunk_px_for(long NP) {
 static void launch_wgrad(const WgK& a0, int nchunks, float* dwb, hipStream_t st) {
     WgK a = a0;
     const int NB = a.cout / 16;
-    const dim3 grd((unsigned)((a.Kext + 63) / 64), (unsigned)nchunks);
+    const dim3 grd((unsigned)((a.Kext + WG_K - 1) / WG_K), (unsigned)nchunks);
     switch (NB) {
         case 2: wgrad_kernel<2><<<grd, 256, 0, st>>>(a); break;
         case 3: wgrad_kernel<3><<<grd, 256, 0, st>>>(a); break;
@@ -719,7 +857,7 @@ static void launch_wgrad(const WgK& a0, int nchunks, float* dwb, hipStream_t st)
         default: break;
     }
     const long n = (long)a.Kext * a.cout;
-    wgrad_reduce_kernel<<<grid_for(n), 256, 0, st>>>(a.part, nchunks, n, dwb);
+    wgrad_reduce_kernel<<<(unsigned)((n + 63) / 64), 256, 0, st>>>(a.part, nchunks, n, dwb);
 }
 
 }  // namespace psw
@@ -735,10 +873,9 @@ struct psw_unet {
     uint16_t* wpb[UN_LAYERS];
     uint16_t* act[UN_LAYERS + 1];
     uint16_t* pool[3];
-    float* gact[UN_LAYERS + 1];
     float* gpool[3];
-    float* tmp = nullptr;
-    uint16_t* dz = nullptr;
+    float* tmp[3];          // data gradients of the concatenated inputs, by level
+    uint16_t* dz[2];        // dZ of the current layer and of the one below
     float *out = nullptr, *gout = nullptr, *tgt = nullptr, *ds = nullptr;
     float* part = nullptr;
     double* lpart = nullptr;
@@ -767,25 +904,18 @@ static int unet_alloc(psw_unet* n, void** p, size_t bytes) {
     return PSW_OK;
 }
 
-// bf16 weight packs of layer L from theta
-static int unet_pack(psw_unet* n, int L, hipStream_t st) {
-    const LayerDef& d = kLayers[L];
-    const int cin = d.ca + d.cb;
-    const int kf = conv_chunks(cin), kb = conv_chunks(d.cout);
-    pack_w_kernel<<<grid_for((long)kf * (d.cout / 16) * 512), 256, 0, st>>>(n->theta + n->off[L], cin, d.cout, 0, kf,
-                                                                            d.cout / 16, n->wpf[L]);
-    if (L > 0)
-        pack_w_kernel<<<grid_for((long)kb * (cin / 16) * 512), 256, 0, st>>>(n->theta + n->off[L], cin, d.cout, 1,
-                                                                             kb, cin / 16, n->wpb[L]);
-    return launch_status("pack_w_kernel");
-}
-
+// bf16 weight packs of all layers from theta
 static int unet_pack_all(psw_unet* n, hipStream_t st) {
+    PackAllK a;
+    int np = 0;
     for (int L = 0; L < UN_LAYERS; ++L) {
-        int s = unet_pack(n, L, st);
-        if (s != PSW_OK) return s;
+        const LayerDef& d = kLayers[L];
+        const int cin = d.ca + d.cb;
+        a.p[np++] = PackK{n->theta + n->off[L], n->wpf[L], cin, d.cout, 0, conv_chunks(cin), d.cout / 16};
+        if (L > 0) a.p[np++] = PackK{n->theta + n->off[L], n->wpb[L], cin, d.cout, 1, conv_chunks(d.cout), cin / 16};
     }
-    return PSW_OK;
+    pack_all_kernel<<<dim3(32, (unsigned)np), 256, 0, st>>>(a);
+    return launch_status("pack_all_kernel");
 }
 
 static int unet_check_shape(psw_unet* n, int batch, int width, int height) {
@@ -816,7 +946,7 @@ static int unet_forward_impl(psw_unet* n, int B, int W, int H, hipStream_t st) {
         a.ca = d.ca; a.cb = d.cb; a.cout = d.cout;
         a.B = B; a.H = H >> d.level; a.W = W >> d.level;
         a.kchunks = conv_chunks(d.ca + d.cb);
-        launch_conv<true>(a, d.cout / 16, st);
+        launch_conv<CONV_RELU>(a, d.cout / 16, st);
         int s = launch_status("conv3x3_kernel");
         if (s != PSW_OK) return s;
         if (L == 1 || L == 3 || L == 5) {
@@ -836,13 +966,15 @@ static int unet_forward_impl(psw_unet* n, int B, int W, int H, hipStream_t st) {
 
 static int unet_backward_impl(psw_unet* n, int B, int W, int H, hipStream_t st) {
     const long NP = (long)B * W * H;
+    int cur = 0;   // dz[cur]: the current layer's dZ
     {
-        const int cpx = chunk_px_for(NP);
-        const int nch = (int)((NP + cpx - 1) / cpx);
-        head_bwd_kernel<<<nch, 256, 0, st>>>(n->act[UN_LAYERS], n->gout, n->theta + n->off[UN_LAYERS], NP, cpx,
-                                             n->gact[UN_LAYERS], n->part);
+        const int cpx = 512;   // chunks enough for several blocks per CU
+        const int nch = (int)std::min<long>((NP + cpx - 1) / cpx, 4096);
+        const int per = (int)((NP + nch - 1) / nch);
+        head_bwd_kernel<<<nch, 256, 0, st>>>(n->act[UN_LAYERS], n->gout, n->theta + n->off[UN_LAYERS], NP, per,
+                                             n->dz[cur], n->part);
         const long nh = UN_HEAD_IN * UN_OUT + UN_OUT;
-        wgrad_reduce_kernel<<<grid_for(nh), 256, 0, st>>>(n->part, nch, nh, n->grad + n->off[UN_LAYERS]);
+        wgrad_reduce_kernel<<<(unsigned)((nh + 63) / 64), 256, 0, st>>>(n->part, nch, nh, n->grad + n->off[UN_LAYERS]);
         int s = launch_status("head_bwd_kernel");
         if (s != PSW_OK) return s;
     }
@@ -850,10 +982,9 @@ static int unet_backward_impl(psw_unet* n, int B, int W, int H, hipStream_t st) 
         const LayerDef& d = kLayers[L];
         const int h = H >> d.level, w = W >> d.level;
         const long np = (long)B * h * w;
-        relu_bwd_kernel<<<grid_for(np * d.cout), 256, 0, st>>>(n->act[L + 1], n->gact[L + 1], n->dz, np * d.cout);
         WgK g;
         layer_inputs(n, L, &g.xa, &g.xb);
-        g.dz = n->dz;
+        g.dz = n->dz[cur];
         g.part = n->part;
         g.ca = d.ca; g.cb = d.cb; g.cout = d.cout;
         g.B = B; g.H = h; g.W = w;
@@ -864,37 +995,35 @@ static int unet_backward_impl(psw_unet* n, int B, int W, int H, hipStream_t st) 
         int s = launch_status("wgrad_kernel");
         if (s != PSW_OK) return s;
         if (L == 0) break;
+        // the data gradient, into the dZ of layer L - 1 (whose output is L's
+        // input, or the coarse half of it, or is pooled into it)
         ConvK a;
-        a.xa = n->dz; a.xb = nullptr; a.wp = n->wpb[L]; a.bias = nullptr;
+        a.xa = n->dz[cur]; a.xb = nullptr; a.wp = n->wpb[L]; a.bias = nullptr; a.mask = nullptr;
         a.ca = d.cout; a.cb = 0; a.cout = d.ca + d.cb;
         a.B = B; a.H = h; a.W = w;
         a.kchunks = conv_chunks(d.cout);
-        static const int dst_a[UN_LAYERS] = {0, 1, -1, 3, -2, 5, -3, 7, 6, 9, 4, 11, 2, 13};
-        if (d.cb == 0) {
-            const int t = dst_a[L];
-            a.y = t >= 0 ? (void*)n->gact[t] : (void*)n->gpool[-t - 1];
-            launch_conv<false>(a, a.cout / 16, st);
-            if ((s = launch_status("conv3x3_kernel (dgrad)")) != PSW_OK) return s;
-            if (t < 0) {
-                // pooled input: distribute into the pooled activation's gradient
-                const int pl = -t - 1;
-                const int src = 2 * pl + 2;  // act index that was pooled (e0, e1, e2)
-                const int lv = kLayers[src - 1].level;
-                const long nfine = (long)B * (H >> lv) * (W >> lv) * kLayers[src - 1].cout;
-                pool_bwd_kernel<<<grid_for(nfine), 256, 0, st>>>(n->gpool[pl], kLayers[src - 1].cout, B, H >> lv,
-                                                                 W >> lv, n->gact[src]);
-                if ((s = launch_status("pool_bwd_kernel")) != PSW_OK) return s;
-            }
+        uint16_t* const next = n->dz[cur ^ 1];
+        const uint16_t* const y = n->act[L];   // output of layer L - 1
+        if (d.cb) {
+            a.y = n->tmp[d.level];
+            launch_conv<CONV_F32>(a, a.cout / 16, st);
+            const long tot = np / 4 * (d.cb / 8);
+            up_bwd_kernel<<<grid_for(tot), 256, 0, st>>>(n->tmp[d.level], d.ca, d.cb, B, h, w, y, next);
+        } else if (L == 2 || L == 4 || L == 6) {
+            const int pl = d.level - 1;
+            const LayerDef& cat = kLayers[12 - 2 * pl];   // the decoder layer that also reads act[L]
+            a.y = n->gpool[pl];
+            launch_conv<CONV_F32>(a, a.cout / 16, st);
+            const long tot = np * 4 * (cat.ca / 8);
+            skip_bwd_kernel<<<grid_for(tot), 256, 0, st>>>(n->tmp[pl], cat.ca, cat.cb, B, 2 * h, 2 * w, n->gpool[pl], y,
+                                                           next);
         } else {
-            a.y = n->tmp;
-            launch_conv<false>(a, a.cout / 16, st);
-            if ((s = launch_status("conv3x3_kernel (dgrad)")) != PSW_OK) return s;
-            static const int dst_b[UN_LAYERS] = {-9, -9, -9, -9, -9, -9, -9, -9, 8, -9, 10, -9, 12, -9};
-            const long tot = np * d.ca + (long)B * (h / 2) * (w / 2) * d.cb;
-            concat_bwd_kernel<<<grid_for(tot), 256, 0, st>>>(n->tmp, d.ca, d.cb, B, h, w, n->gact[dst_a[L]],
-                                                             n->gact[dst_b[L]]);
-            if ((s = launch_status("concat_bwd_kernel")) != PSW_OK) return s;
+            a.mask = y;
+            a.y = next;
+            launch_conv<CONV_MASKED>(a, a.cout / 16, st);
         }
+        if ((s = launch_status("data gradient")) != PSW_OK) return s;
+        cur ^= 1;
     }
     return PSW_OK;
 }
@@ -925,8 +1054,8 @@ int psw_unet_create(psw_unet** out, int64_t max_pixels) {
     A((void**)&n->grad, P * 4);
     A((void**)&n->m, P * 4);
     A((void**)&n->v, P * 4);
-    size_t part_floats = (size_t)257 * (UN_HEAD_IN * UN_OUT + UN_OUT);
-    size_t tmp_floats = 0, dz_el = 0;
+    size_t part_floats = (size_t)4097 * (UN_HEAD_IN * UN_OUT + UN_OUT);
+    size_t dz_el = 0;
     for (int L = 0; L < UN_LAYERS; ++L) {
         const LayerDef& d = kLayers[L];
         const int cin = d.ca + d.cb;
@@ -934,21 +1063,19 @@ int psw_unet_create(psw_unet** out, int64_t max_pixels) {
         A((void**)&n->wpb[L], (size_t)conv_chunks(d.cout) * (cin / 16) * 512 * 2);
         const size_t np = (size_t)(max_pixels >> (2 * d.level));
         A((void**)&n->act[L + 1], np * d.cout * 2);
-        A((void**)&n->gact[L + 1], np * d.cout * 4);
         part_floats = std::max(part_floats, (size_t)257 * (9 * cin + 1) * d.cout);
-        if (d.cb) tmp_floats = std::max(tmp_floats, np * cin);
+        if (d.cb) A((void**)&n->tmp[d.level], np * cin * 4);
         dz_el = std::max(dz_el, np * d.cout);
     }
     A((void**)&n->act[0], (size_t)max_pixels * UN_IN * 2);
-    n->gact[0] = nullptr;
     for (int pl = 0; pl < 3; ++pl) {
         const int c = kLayers[2 * pl + 1].cout;
         const size_t np = (size_t)(max_pixels >> (2 * (pl + 1)));
         A((void**)&n->pool[pl], np * c * 2);
         A((void**)&n->gpool[pl], np * c * 4);
     }
-    A((void**)&n->tmp, tmp_floats * 4);
-    A((void**)&n->dz, dz_el * 2);
+    A((void**)&n->dz[0], dz_el * 2);
+    A((void**)&n->dz[1], dz_el * 2);
     A((void**)&n->out, (size_t)max_pixels * UN_OUT * 4);
     A((void**)&n->gout, (size_t)max_pixels * UN_OUT * 4);
     A((void**)&n->tgt, (size_t)max_pixels * UN_OUT * 4);
@@ -1155,12 +1282,12 @@ int psw_conv3x3_bf16(const uint16_t* d_xa, int ca, const uint16_t* d_xb, int cb,
     uint16_t* wp = nullptr;
     PSW_TRY_HIP(hipMalloc((void**)&wp, (size_t)kc * (cout / 16) * 512 * 2), PSW_ERR_ALLOC);
     hipStream_t st = S(s);
-    pack_w_kernel<<<grid_for((long)kc * (cout / 16) * 512), 256, 0, st>>>(d_w, cin, cout, 0, kc, cout / 16, wp);
+    pack_w_kernel<<<grid_for((long)kc * (cout / 16) * 512), 256, 0, st>>>(PackK{d_w, wp, cin, cout, 0, kc, cout / 16});
     ConvK a;
     a.xa = d_xa; a.xb = d_xb; a.wp = wp; a.bias = d_bias; a.y = d_y;
     a.ca = ca; a.cb = cb; a.cout = cout; a.B = batch; a.H = height; a.W = width; a.kchunks = kc;
-    if (relu_bf16) launch_conv<true>(a, cout / 16, st);
-    else launch_conv<false>(a, cout / 16, st);
+    if (relu_bf16) launch_conv<CONV_RELU>(a, cout / 16, st);
+    else launch_conv<CONV_F32>(a, cout / 16, st);
     int r = launch_status("conv3x3_kernel");
     (void)hipStreamSynchronize(st);
     (void)hipFree(wp);
@@ -1176,11 +1303,11 @@ int psw_conv3x3_bf16_dgrad(const uint16_t* d_dz, int cout, const float* d_w, int
     uint16_t* wp = nullptr;
     PSW_TRY_HIP(hipMalloc((void**)&wp, (size_t)kc * (cin / 16) * 512 * 2), PSW_ERR_ALLOC);
     hipStream_t st = S(s);
-    pack_w_kernel<<<grid_for((long)kc * (cin / 16) * 512), 256, 0, st>>>(d_w, cin, cout, 1, kc, cin / 16, wp);
+    pack_w_kernel<<<grid_for((long)kc * (cin / 16) * 512), 256, 0, st>>>(PackK{d_w, wp, cin, cout, 1, kc, cin / 16});
     ConvK a;
     a.xa = d_dz; a.xb = nullptr; a.wp = wp; a.bias = nullptr; a.y = d_dx;
     a.ca = cout; a.cb = 0; a.cout = cin; a.B = batch; a.H = height; a.W = width; a.kchunks = kc;
-    launch_conv<false>(a, cin / 16, st);
+    launch_conv<CONV_F32>(a, cin / 16, st);
     int r = launch_status("conv3x3_kernel (dgrad)");
     (void)hipStreamSynchronize(st);
     (void)hipFree(wp);
