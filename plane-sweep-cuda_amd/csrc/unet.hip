@@ -76,7 +76,10 @@ struct ConvK {
     const uint16_t* wp;   // packed weights [conv_chunks(ca + cb)][NB][64][8]
     const float* bias;    // [cout] or null
     const uint16_t* mask; // [B][H][W][cout] activations (CONV_MASKED)
-    void* y;              // [B][H][W][cout]: bf16 or fp32, see ConvOut
+    void* y;              // [B][H][W][cout]: bf16 or fp32, see ConvOut; CONV_HEAD: may be null
+    uint16_t* pool;       // CONV_POOL: the 2x2 average pool, [B][H/2][W/2][cout]
+    const float* head;    // CONV_HEAD (blocks of all cout = UN_HEAD_IN channels): the head's weights
+    float* head_out;      // and its output [B][H][W][UN_OUT]
     int ca, cb, cout, B, H, W, kchunks;
 };
 
@@ -85,7 +88,10 @@ struct ConvK {
 // gradient that goes straight on to the layer below as its dZ: FP32
 // gradients and a pass over them to mask and round (19 us on average, ten
 // times per training step of 8 x 256 x 256) never reach memory.
-enum ConvOut { CONV_F32, CONV_RELU, CONV_MASKED };
+// CONV_POOL and CONV_HEAD are CONV_RELU that also writes the average pool or
+// the head's output (forms of their own: the head's registers would cost
+// every ReLU layer a wave per SIMD, 30 us a launch at 640 x 480 instead of 23).
+enum ConvOut { CONV_F32, CONV_RELU, CONV_MASKED, CONV_POOL, CONV_HEAD };
 
 // Output tile of one block: 8 rows x 32 columns, four waves of 2 rows each
 // (4 MFMA row blocks of 16 pixels per wave).  The input tile with its
@@ -162,11 +168,25 @@ __device__ __forceinline__ void conv_slab(f32x4 (&acc)[4][NBL], const uint16_t* 
     }
 }
 
+// Adds 16 channels of a pixel to its head outputs, in channel order (the
+// head's weights are uniform: scalar loads).
+__device__ __forceinline__ void head_add(float (&o)[UN_OUT], uint4 v0, uint4 v1, const float* __restrict__ w) {
+    const uint32_t d[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+        const float xv = bf2f((uint16_t)(d[c >> 1] >> (16 * (c & 1))));
+#pragma unroll
+        for (int k = 0; k < UN_OUT; ++k) o[k] += xv * w[c * UN_OUT + k];
+    }
+}
+
 // A block computes NBL of the layer's nbtot 16-channel output blocks
 // (starting at blockIdx.y * NBL): small levels split their output channels
 // over several blocks so that a launch still has enough of them.  The
 // results go through LDS, 16 channels at a time, so that every thread
-// stores whole 16-byte runs of one pixel's channels.
+// stores whole 16-byte runs of one pixel's channels.  From there the 2x2
+// average pool of the tile and, for the last layer, the 1x1 head cost no
+// pass over the activations of their own (640 x 480: 23 and 10 us).
 template <int NBL, int OUT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NBL == 1 ? 4 : 1)))
 void conv3x3_kernel(ConvK a) {
@@ -275,6 +295,11 @@ void conv3x3_kernel(ConvK a) {
     const int y = ty0 + ty, x = tx0 + tx;
     const long p = ((long)b * a.H + y) * a.W + x;
     const bool out = y < a.H && x < a.W;
+    float o[UN_OUT];   // the head's output of this thread's pixel
+    if (OUT == CONV_HEAD) {
+#pragma unroll
+        for (int k = 0; k < UN_OUT; ++k) o[k] = a.head[UN_HEAD_IN * UN_OUT + k];
+    }
 #pragma unroll
     for (int nb = 0; nb < NBL; ++nb) {
         const int ch0 = (nb0 + nb) * 16;
@@ -287,20 +312,45 @@ void conv3x3_kernel(ConvK a) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int q = (wave * 2 + (m >> 1)) * CT_TW + (m & 1) * 16 + 4 * jg + i;
-                    so[q * 24 + col] = f2bf(OUT == CONV_RELU ? fmaxf(acc[m][nb][i] + bias, 0.f) : acc[m][nb][i]);
+                    so[q * 24 + col] = f2bf(OUT == CONV_MASKED ? acc[m][nb][i] : fmaxf(acc[m][nb][i] + bias, 0.f));
                 }
             __syncthreads();
             if (out) {
                 const uint4* src = reinterpret_cast<const uint4*>(&so[t * 24]);
-                uint4* dst = reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(a.y) + p * a.cout + ch0);
                 uint4 v0 = src[0], v1 = src[1];
                 if (OUT == CONV_MASKED) {
                     const uint4* mk = reinterpret_cast<const uint4*>(a.mask + p * a.cout + ch0);
                     v0 = mask_bf16x8(v0, mk[0]);
                     v1 = mask_bf16x8(v1, mk[1]);
                 }
-                dst[0] = v0;
-                dst[1] = v1;
+                if (OUT != CONV_HEAD || a.y) {
+                    uint4* dst = reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(a.y) + p * a.cout + ch0);
+                    dst[0] = v0;
+                    dst[1] = v1;
+                }
+                if constexpr (OUT == CONV_HEAD) head_add(o, v0, v1, a.head + ch0 * UN_OUT);
+            }
+            if (OUT == CONV_POOL && t < CT_TH / 2 * (CT_TW / 2) * 2) {
+                // pooled pixel t / 2 of the tile, 8 of the 16 channels
+                const int q = t >> 1, py = q / (CT_TW / 2), px = q - py * (CT_TW / 2), cg = (t & 1) * 8;
+                const int gy = (ty0 >> 1) + py, gx = (tx0 >> 1) + px;
+                if (gy < Hh && gx < Wh) {
+                    const uint16_t* s00 = &so[(2 * py * CT_TW + 2 * px) * 24 + cg];
+                    uint32_t d[4];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        float e[2];
+#pragma unroll
+                        for (int k = 0; k < 2; ++k) {
+                            const int i = 2 * c + k;
+                            e[k] = 0.25f * ((bf2f(s00[i]) + bf2f(s00[24 + i])) +
+                                            (bf2f(s00[CT_TW * 24 + i]) + bf2f(s00[CT_TW * 24 + 24 + i])));
+                        }
+                        d[c] = pack_bf16x2(e[0], e[1]);
+                    }
+                    *reinterpret_cast<uint4*>(a.pool + (((long)b * Hh + gy) * Wh + gx) * a.cout + ch0 + cg) =
+                        make_uint4(d[0], d[1], d[2], d[3]);
+                }
             }
         } else {
             float* so = reinterpret_cast<float*>(sx);
@@ -318,6 +368,13 @@ void conv3x3_kernel(ConvK a) {
 #pragma unroll
                 for (int k = 0; k < 4; ++k) dst[k] = src[k];
             }
+        }
+    }
+    if constexpr (OUT == CONV_HEAD) {
+        if (out) {
+            float4* dst = reinterpret_cast<float4*>(a.head_out + p * UN_OUT);
+            dst[0] = make_float4(o[0], o[1], o[2], o[3]);
+            dst[1] = make_float4(o[4], o[5], o[6], o[7]);
         }
     }
 }
@@ -387,7 +444,8 @@ struct WgK {
 // Chunk partials are summed in a fixed order by wgrad_reduce_kernel
 // (deterministic).
 // Bound by the transposition's LDS traffic and by latency, not by the matrix
-// cores: WGRAD_FIGURES
+// cores.  8 x 256 x 256: the level-0 layers 70 us on average, against 113 with
+// 32 pixels per step and 2-byte transposing stores.
 constexpr int WG_PX = 128, WG_ST = WG_PX + 8, WG_MR = 2, WG_K = 64 * WG_MR;
 
 // 4 pixels x 8 channels -> per channel, its 4 pixels.
@@ -528,7 +586,7 @@ __global__ __launch_bounds__(256) void wgrad_kernel(WgK a) {
 // Sums the chunks' partials in a fixed order: four waves take a quarter of
 // the chunks each for 64 entries, eight loads in flight, then add up.  (One
 // thread per entry walking all chunks had too few threads to hide its
-// loads: 42 us a call on average, now REDUCE_FIGURES.)
+// loads: 42 us a call on average at 8 x 256 x 256, now 7.)
 __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float* __restrict__ part, int nchunks, long n,
                                                            float* __restrict__ out) {
     __shared__ float ss[4][64];
@@ -602,22 +660,6 @@ __global__ void skip_bwd_kernel(const float* __restrict__ tmp, int ca, int cb, i
     }
 }
 
-// 2x2 average pooling (bf16 -> bf16, FP32 sum).
-__global__ void pool_fwd_kernel(const uint16_t* __restrict__ x, int C, int B, int H, int W, uint16_t* __restrict__ y) {
-    const int Hh = H >> 1, Wh = W >> 1;
-    const long n = (long)B * Hh * Wh * C;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        const long q = i / C;
-        const int c = (int)(i - q * C);
-        const int xx = (int)(q % Wh);
-        const long tt = q / Wh;
-        const int yy = (int)(tt % Hh), b = (int)(tt / Hh);
-        const long p = ((long)b * H + 2 * yy) * W + 2 * xx;
-        const float s = (bf2f(x[p * C + c]) + bf2f(x[(p + 1) * C + c])) + (bf2f(x[(p + W) * C + c]) + bf2f(x[(p + W + 1) * C + c]));
-        y[i] = f2bf(0.25f * s);
-    }
-}
-
 // Head: out[p][o] = b[o] + sum_c d0[p][c] W[c][o] (FP32).
 __global__ void head_fwd_kernel(const uint16_t* __restrict__ x, const float* __restrict__ w, long NP,
                                 float* __restrict__ out) {
@@ -648,49 +690,75 @@ __global__ void head_fwd_kernel(const uint16_t* __restrict__ x, const float* __r
 // Head backward: dZ of the last layer from g_x[p][c] = sum_o g[p][o] W[c][o]
 // (masked by x > 0, bf16); per-chunk partials of
 // dW[c][o] = sum_p x[p][c] g[p][o] and db[o] = sum_p g[p][o].
+// 64 pixels per step.  Bound by LDS reads, so the products are register
+// tiles: a thread forms 8 channels of one pixel's g_x from 8 reads (its part
+// of W stays in registers), and 2 x 2 entries of dW per pixel from 4, each
+// wave on a quarter of the pixels.  8 x 256 x 256: 20 us, against
+// 163 with one entry of dW and one channel of g_x per thread.
+constexpr int HB_PX = 64;
 __global__ __launch_bounds__(256) void head_bwd_kernel(const uint16_t* __restrict__ x, const float* __restrict__ g,
                                                        const float* __restrict__ w, long NP, int chunk_px,
                                                        uint16_t* __restrict__ dz, float* __restrict__ part) {
-    __shared__ float sw[UN_HEAD_IN * UN_OUT];
-    __shared__ float sx[64][UN_HEAD_IN + 1];
-    __shared__ float sg[64][UN_OUT + 1];
-    const int t = threadIdx.x;
-    for (int i = t; i < UN_HEAD_IN * UN_OUT; i += 256) sw[i] = w[i];
+    constexpr int NW = UN_HEAD_IN * UN_OUT;
+    __shared__ float sx[HB_PX][UN_HEAD_IN + 1];
+    __shared__ __align__(16) float sg[HB_PX][UN_OUT + 4];
+    __shared__ float sp[4][NW + UN_OUT];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const long p_begin = (long)blockIdx.x * chunk_px;
     const long p_end = p_begin + chunk_px < NP ? p_begin + chunk_px : NP;
-    const int c = t >> 3, o = t & 7;  // this thread's dW entry
-    float accw = 0.f, accb = 0.f;
-    __syncthreads();
-    for (long p0 = p_begin; p0 < p_end; p0 += 64) {
-        // stage 64 pixels of x and g
-        for (int i = t; i < 64 * UN_HEAD_IN; i += 256) {
-            const long p = p0 + i / UN_HEAD_IN;
-            sx[i / UN_HEAD_IN][i % UN_HEAD_IN] = p < p_end ? bf2f(x[p * UN_HEAD_IN + i % UN_HEAD_IN]) : 0.f;
-        }
-        for (int i = t; i < 64 * UN_OUT; i += 256) {
-            const long p = p0 + i / UN_OUT;
-            sg[i / UN_OUT][i % UN_OUT] = p < p_end ? g[p * UN_OUT + i % UN_OUT] : 0.f;
-        }
-        __syncthreads();
-        for (int r = 0; r < 64; ++r) accw += sx[r][c] * sg[r][o];
-        if (t < UN_OUT)
-            for (int r = 0; r < 64; ++r) accb += sg[r][t];
-        // g_x for these pixels: thread handles (pixel r, channel pair)
-        for (int i = t; i < 64 * UN_HEAD_IN; i += 256) {
-            const int r = i / UN_HEAD_IN, cc = i % UN_HEAD_IN;
-            const long p = p0 + r;
-            if (p < p_end) {
-                float s = 0.f;
+    const int r = t >> 2, c8 = (t & 3) * 8;                  // this thread's pixel and channels of x and g_x
+    const int c2 = (lane >> 2) * 2, o2 = (lane & 3) * 2;     // its dW entries
+    float rw[8][UN_OUT];
 #pragma unroll
-                for (int k = 0; k < UN_OUT; ++k) s += sg[r][k] * sw[cc * UN_OUT + k];
-                dz[p * UN_HEAD_IN + cc] = sx[r][cc] > 0.f ? f2bf(s) : (uint16_t)0;
+    for (int c = 0; c < 8; ++c)
+#pragma unroll
+        for (int o = 0; o < UN_OUT; ++o) rw[c][o] = w[(c8 + c) * UN_OUT + o];
+    float a00 = 0.f, a01 = 0.f, a10 = 0.f, a11 = 0.f, accb = 0.f;
+    for (long p0 = p_begin; p0 < p_end; p0 += HB_PX) {
+        const long p = p0 + r;
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);
+        if (p < p_end) v = *reinterpret_cast<const uint4*>(x + p * UN_HEAD_IN + c8);
+        float2 gv = make_float2(0.f, 0.f);
+        if (p < p_end) gv = *reinterpret_cast<const float2*>(g + p * UN_OUT + (t & 3) * 2);
+        __syncthreads();   // the previous step's reads are done
+        const uint16_t* e = reinterpret_cast<const uint16_t*>(&v);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) sx[r][c8 + c] = bf2f(e[c]);
+        *reinterpret_cast<float2*>(&sg[r][(t & 3) * 2]) = gv;
+        __syncthreads();
+        {
+            float gr[UN_OUT];
+#pragma unroll
+            for (int o = 0; o < UN_OUT; ++o) gr[o] = sg[r][o];
+            float s[8];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                s[c] = 0.f;
+#pragma unroll
+                for (int o = 0; o < UN_OUT; ++o) s[c] += gr[o] * rw[c][o];
+            }
+            if (p < p_end) {
+                const uint4 d = make_uint4(pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3]), pack_bf16x2(s[4], s[5]),
+                                           pack_bf16x2(s[6], s[7]));
+                *reinterpret_cast<uint4*>(dz + p * UN_HEAD_IN + c8) = mask_bf16x8(d, v);
             }
         }
-        __syncthreads();
+#pragma unroll 4
+        for (int q = wave * (HB_PX / 4); q < (wave + 1) * (HB_PX / 4); ++q) {
+            const float x0 = sx[q][c2], x1 = sx[q][c2 + 1], g0 = sg[q][o2], g1 = sg[q][o2 + 1];
+            a00 += x0 * g0; a01 += x0 * g1;
+            a10 += x1 * g0; a11 += x1 * g1;
+            if (lane < UN_OUT) accb += sg[q][lane];
+        }
     }
-    float* pp = part + (long)blockIdx.x * (UN_HEAD_IN * UN_OUT + UN_OUT);
-    pp[c * UN_OUT + o] = accw;
-    if (t < UN_OUT) pp[UN_HEAD_IN * UN_OUT + t] = accb;
+    sp[wave][c2 * UN_OUT + o2] = a00;
+    sp[wave][c2 * UN_OUT + o2 + 1] = a01;
+    sp[wave][(c2 + 1) * UN_OUT + o2] = a10;
+    sp[wave][(c2 + 1) * UN_OUT + o2 + 1] = a11;
+    if (lane < UN_OUT) sp[wave][NW + lane] = accb;
+    __syncthreads();
+    float* pp = part + (long)blockIdx.x * (NW + UN_OUT);
+    for (int i = t; i < NW + UN_OUT; i += 256) pp[i] = (sp[0][i] + sp[1][i]) + (sp[2][i] + sp[3][i]);
 }
 
 // Smooth-L1 (Huber, delta 1) loss per channel with weights wc; g = dL/dout.
@@ -816,13 +884,25 @@ static inline unsigned grid_for(long n, int per = 256) {
 
 // Output-channel split: levels with few tiles give each block fewer
 // 16-channel output blocks (NBL), so that a launch has about 1000 blocks.
-template <int OUT>
-static void launch_conv(const ConvK& a, int NB, hipStream_t st) {
-    const long tiles = (long)a.B * ((a.H + CT_TH - 1) / CT_TH) * ((a.W + CT_TW - 1) / CT_TW);
+static long conv_tiles(const ConvK& a) {
+    return (long)a.B * ((a.H + CT_TH - 1) / CT_TH) * ((a.W + CT_TW - 1) / CT_TW);
+}
+static int conv_nbl(const ConvK& a, int NB) {
+    const long tiles = conv_tiles(a);
     int nbl = NB;
     if (tiles * 2 < 1024 && NB % 2 == 0 && NB > 2) nbl = 2;
     if (tiles * (NB / nbl) < 1024) nbl = 1;
+    return nbl;
+}
+template <int OUT>
+static void launch_conv(const ConvK& a, int NB, hipStream_t st) {
+    const long tiles = conv_tiles(a);
+    const int nbl = conv_nbl(a, NB);
     const dim3 grd((unsigned)tiles, (unsigned)(NB / nbl));
+    if constexpr (OUT == CONV_HEAD) {   // two output blocks per block
+        conv3x3_kernel<2, OUT><<<grd, 256, 0, st>>>(a);
+        return;
+    }
     switch (nbl) {
 #define PSW_CONV_CASE(n) \
     case n: conv3x3_kernel<n, OUT><<<grd, 256, 0, st>>>(a); break;
@@ -935,10 +1015,12 @@ static void layer_inputs(psw_unet* n, int L, const uint16_t** xa, const uint16_t
     *xb = src_b[L] >= 0 ? n->act[src_b[L]] : nullptr;
 }
 
-static int unet_forward_impl(psw_unet* n, int B, int W, int H, hipStream_t st) {
+// train: keep the last layer's activations for the backward pass
+static int unet_forward_impl(psw_unet* n, int B, int W, int H, bool train, hipStream_t st) {
+    bool head = false;
     for (int L = 0; L < UN_LAYERS; ++L) {
         const LayerDef& d = kLayers[L];
-        ConvK a;
+        ConvK a = {};
         layer_inputs(n, L, &a.xa, &a.xb);
         a.wp = n->wpf[L];
         a.bias = n->theta + n->off[L] + (size_t)9 * (d.ca + d.cb) * d.cout;
@@ -946,18 +1028,22 @@ static int unet_forward_impl(psw_unet* n, int B, int W, int H, hipStream_t st) {
         a.ca = d.ca; a.cb = d.cb; a.cout = d.cout;
         a.B = B; a.H = H >> d.level; a.W = W >> d.level;
         a.kchunks = conv_chunks(d.ca + d.cb);
-        launch_conv<CONV_RELU>(a, d.cout / 16, st);
+        if (L == 1 || L == 3 || L == 5) {
+            a.pool = n->pool[(L - 1) / 2];
+            launch_conv<CONV_POOL>(a, d.cout / 16, st);
+        } else if (L == UN_LAYERS - 1 && conv_nbl(a, d.cout / 16) * 16 == UN_HEAD_IN) {
+            head = true;
+            a.head = n->theta + n->off[UN_LAYERS];
+            a.head_out = n->out;
+            if (!train) a.y = nullptr;
+            launch_conv<CONV_HEAD>(a, d.cout / 16, st);
+        } else {
+            launch_conv<CONV_RELU>(a, d.cout / 16, st);
+        }
         int s = launch_status("conv3x3_kernel");
         if (s != PSW_OK) return s;
-        if (L == 1 || L == 3 || L == 5) {
-            const int pl = (L - 1) / 2;
-            const long np = (long)B * (H >> (d.level + 1)) * (W >> (d.level + 1)) * d.cout;
-            pool_fwd_kernel<<<grid_for(np), 256, 0, st>>>(n->act[L + 1], d.cout, B, H >> d.level, W >> d.level,
-                                                          n->pool[pl]);
-            s = launch_status("pool_fwd_kernel");
-            if (s != PSW_OK) return s;
-        }
     }
+    if (head) return PSW_OK;
     const long NP = (long)B * W * H;
     head_fwd_kernel<<<(unsigned)((NP + 255) / 256), 256, 0, st>>>(n->act[UN_LAYERS], n->theta + n->off[UN_LAYERS], NP,
                                                                   n->out);
@@ -997,7 +1083,7 @@ static int unet_backward_impl(psw_unet* n, int B, int W, int H, hipStream_t st) 
         if (L == 0) break;
         // the data gradient, into the dZ of layer L - 1 (whose output is L's
         // input, or the coarse half of it, or is pooled into it)
-        ConvK a;
+        ConvK a = {};
         a.xa = n->dz[cur]; a.xb = nullptr; a.wp = n->wpb[L]; a.bias = nullptr; a.mask = nullptr;
         a.ca = d.cout; a.cb = 0; a.cout = d.ca + d.cb;
         a.B = B; a.H = h; a.W = w;
@@ -1194,7 +1280,7 @@ int psw_unet_set_target(psw_unet* n, int slot, int width, int height, const floa
 int psw_unet_forward(psw_unet* n, int batch, int width, int height, psw_stream_t s) {
     int st = unet_check_shape(n, batch, width, height);
     if (st != PSW_OK) return st;
-    return unet_forward_impl(n, batch, width, height, S(s));
+    return unet_forward_impl(n, batch, width, height, false, S(s));
 }
 
 int psw_unet_output(psw_unet* n, int slot, int width, int height, float* d_out, psw_stream_t s) {
@@ -1223,7 +1309,7 @@ int psw_unet_loss_grad(psw_unet* n, int batch, int width, int height, const floa
     if (st != PSW_OK) return st;
     PSW_CHECK_ARG(channel_weights, "NULL channel weights");
     hipStream_t hs = S(s);
-    if ((st = unet_forward_impl(n, batch, width, height, hs)) != PSW_OK) return st;
+    if ((st = unet_forward_impl(n, batch, width, height, true, hs)) != PSW_OK) return st;
     LossK a;
     a.out = n->out; a.tgt = n->tgt; a.g = n->gout; a.part = n->lpart;
     a.NP = (long)batch * width * height;
@@ -1283,7 +1369,7 @@ int psw_conv3x3_bf16(const uint16_t* d_xa, int ca, const uint16_t* d_xb, int cb,
     PSW_TRY_HIP(hipMalloc((void**)&wp, (size_t)kc * (cout / 16) * 512 * 2), PSW_ERR_ALLOC);
     hipStream_t st = S(s);
     pack_w_kernel<<<grid_for((long)kc * (cout / 16) * 512), 256, 0, st>>>(PackK{d_w, wp, cin, cout, 0, kc, cout / 16});
-    ConvK a;
+    ConvK a = {};
     a.xa = d_xa; a.xb = d_xb; a.wp = wp; a.bias = d_bias; a.y = d_y;
     a.ca = ca; a.cb = cb; a.cout = cout; a.B = batch; a.H = height; a.W = width; a.kchunks = kc;
     if (relu_bf16) launch_conv<CONV_RELU>(a, cout / 16, st);
@@ -1304,7 +1390,7 @@ int psw_conv3x3_bf16_dgrad(const uint16_t* d_dz, int cout, const float* d_w, int
     PSW_TRY_HIP(hipMalloc((void**)&wp, (size_t)kc * (cin / 16) * 512 * 2), PSW_ERR_ALLOC);
     hipStream_t st = S(s);
     pack_w_kernel<<<grid_for((long)kc * (cin / 16) * 512), 256, 0, st>>>(PackK{d_w, wp, cin, cout, 1, kc, cin / 16});
-    ConvK a;
+    ConvK a = {};
     a.xa = d_dz; a.xb = nullptr; a.wp = wp; a.bias = nullptr; a.y = d_dx;
     a.ca = cout; a.cb = 0; a.cout = cin; a.B = batch; a.H = height; a.W = width; a.kchunks = kc;
     launch_conv<CONV_F32>(a, cin / 16, st);
