@@ -923,7 +923,7 @@ int psw_sweep_fused_reference(const float* d_ref, const float* d_src, int width,
     // capture, for one source in few planes, or when the pool has no memory.
     const size_t npix = (size_t)width * height;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    (void)hipStreamIsCapturing(S(s), &cap);
+    if (hipStreamIsCapturing(S(s), &cap) != hipSuccess) (void)hipGetLastError();
     void* ws = nullptr;
     const int G = (int)std::max(1L, std::min((long)nplanes, SW_TARGET_ITEMS / ((long)a.ntiles * nsrc)));
     if (cap == hipStreamCaptureStatusNone && nsrc * G > 1 &&
