@@ -1,0 +1,70 @@
+"""The network's launches at the sizes where they can go wrong: the output
+head in the last convolution's epilogue (1024 tiles and more) against the
+separate head kernel, and the weight gradient at odd and tiny widths and over
+several 512-pixel chunks."""
+import numpy as np
+import pytest
+
+from unet_ref import bf16_bits, bf16_val, wgrad_ref
+
+pytestmark = pytest.mark.gpu
+
+
+# 8 x 32 pixels per tile: 18 tiles of a 64 x 72 image, so 56 images make 1008
+# tiles and 57 make 1026.  The first image's outputs differ in the order of
+# the head's 32 products only: 32 roundings of partial sums, each at most 2^-24
+# of the sum of the terms' magnitudes on either side; that sum is bounded here
+# by 64 times the largest output.
+@pytest.mark.parametrize("B", [56, 57])
+def test_head_in_the_epilogue_matches_the_head_kernel(gpu, B):
+    from psw_amd import warmstart
+    from psw_amd.device import DeviceArray
+    W, H = 64, 72
+    rng = np.random.default_rng(5)
+    x = rng.uniform(-1, 1, (H, W, 8)).astype(np.float32)
+    x[..., 5:] = 0
+    net = warmstart.UNet(B * W * H, seed=3)
+    p = net.get_params()
+    p[-264:-8] = rng.standard_normal(256).astype(np.float32) * 0.3
+    net.set_params(p)
+    d_x = DeviceArray.from_host(x)
+    d_d = DeviceArray.from_host(rng.uniform(1.0, 4.0, (H, W)).astype(np.float32))
+    outs = []
+    for n in (1, B):
+        for b in range(n):
+            net.set_input(b, W, H, d_x, d_d)
+        print(f"[case] network forward, {n} images of {W}x{H}", flush=True)
+        net.forward(n, W, H)
+        outs.append([net.output(b, W, H).to_host() for b in (0, n - 1)])
+    one = outs[0][0]
+    tol = 2 * 32 * 2.0 ** -24 * 64 * np.abs(one).max()
+    for o in outs[1]:
+        assert np.abs(o - one).max() <= tol
+
+
+@pytest.mark.parametrize("ca,cb,cout,B,H,W", [(48, 0, 48, 3, 37, 29), (32, 0, 32, 2, 3, 130), (64, 96, 64, 5, 12, 2),
+                                              (8, 0, 32, 7, 41, 3)])
+def test_weight_gradient_at_odd_widths(gpu, ca, cb, cout, B, H, W):
+    from psw_amd._lib import call
+    from psw_amd.device import DeviceArray
+    rng = np.random.default_rng(ca + W)
+    dev = DeviceArray.from_host
+    xa = bf16_bits(rng.standard_normal((B, H, W, ca)))
+    xb = bf16_bits(rng.standard_normal((B, H // 2, W // 2, cb))) if cb else None
+    dz = bf16_bits(rng.standard_normal((B, H, W, cout)))
+    x = bf16_val(xa).astype(np.float64)
+    if cb:
+        up = bf16_val(xb).astype(np.float64).repeat(2, axis=1).repeat(2, axis=2)
+        x = np.concatenate([x, up], axis=3)
+    z = bf16_val(dz).astype(np.float64)
+    dw, db = wgrad_ref(x, z)
+    mw, mb = wgrad_ref(np.abs(x), np.abs(z))
+    d_xa, d_dz, d_xb = dev(xa), dev(dz), dev(xb) if cb else None
+    out = DeviceArray(((9 * (ca + cb) + 1) * cout,))
+    print(f"[case] weight gradient {ca}+{cb}->{cout}, {B} x {H} x {W}", flush=True)
+    call("psw_conv3x3_bf16_wgrad", d_xa.ptr, ca, d_xb.ptr if cb else None, cb, d_dz.ptr, cout, B, W, H, out.ptr, None)
+    g = out.to_host()
+    n = 9 * (ca + cb) * cout
+    # FP32 sums: 1e-5 of the terms' magnitudes, as for the other sizes
+    assert np.all(np.abs(g[:n].reshape(dw.shape) - dw) <= 1e-5 * mw + 1e-6)
+    assert np.all(np.abs(g[n:] - db) <= 1e-5 * mb + 1e-6)
